@@ -15,10 +15,13 @@
 // Small matrices (up to 262144 super-blocks) take gemv_lat_kernel instead:
 // four lanes per super-block, loads straight into registers, one pass.
 //
+// Several tokens take int8 matrix cores (gemv_mt_kernel, gemv_mtw_kernel).
+//
 // Reference kernels replaced: gemv_q4_k_q8 / gemv_mtok_ro_f32_kernel
 // (q4_k.cu:57-91, 1360-1422, 1534-1562), gemv_q4_k_q8_batched and the mtok
 // variants (q4_k.cu:218-282, 359-498), gemv_ptrs_q4_k_q8_f16out
 // (q4_k.cu:184-213).
+#include <algorithm>
 #include <type_traits>
 
 #include "sg_common.hpp"
@@ -26,7 +29,7 @@
 namespace sg {
 
 constexpr int kMaxNb = 64;       // k <= 16384
-constexpr int kMaxTokens = 16;   // batched GEMV token tile
+constexpr int kMaxTokens = 16;   // batched GEMV: the rows of an MFMA result
 constexpr int kWaves = 4;        // waves per workgroup
 constexpr int kBufWords = 64 * 36;  // one wave's 9216-B weight buffer
 constexpr int kWgPerCu = 2;        // grid cap: workgroups per CU
@@ -309,8 +312,10 @@ __global__ void __launch_bounds__(64 * kLatWaves) gemv_lat_plain_kernel(
   gemv_lat_body(PlainRows{w, nb}, xq, F32Out{y}, n_rows, nb, lg);
 }
 
-// y[t*n_rows + r] = W[r] . x[t] for t < n_tokens; weights read once.  The
-// row result goes out through Out (fp32, or rounded to fp16).
+// y[t*n_rows + r] = W[r] . x[t] for the few tokens of short rows
+// (n_tokens * nb <= 8) in large matrices: a lane per super-block as in
+// gemv1_kernel, looping over the tokens with sdot4.  The matrix-core kernels
+// below win everywhere else.
 template <typename Out>
 __global__ void __launch_bounds__(256) gemv_batched_kernel(const sg_block_q4k* __restrict__ w,
                                                            const unsigned char* __restrict__ xq,
@@ -357,6 +362,298 @@ __global__ void __launch_bounds__(256) gemv_batched_kernel(const sg_block_q4k* _
       if (blk == nb - 1 && rr < n) y.store(t * n_rows + r0 + rr, acc);
     }
   }
+}
+
+// y[t*n_rows + r] = W[r] . x[t] for up to 16 tokens on int8 matrix cores, the
+// weights read once; the row result goes out through Out (fp32, or rounded to
+// fp16).  One v_mfma_i32_16x16x32_i8 is one Q4_K sub-block (K = 32) of 16
+// weight rows (columns) against 16 token rows, so every int32 sub-block dot
+// comes out by itself and the fp32 epilogue keeps the GEMV family's order
+// (block_sum, then the block sums added in block order): the same bits.  Wave
+// w owns super-block w of every row, so its activation operands stay in
+// registers, and the block sums of a row meet in LDS, added in block order by
+// one thread per output.
+constexpr int kMtBsWords = 12;  // staged per (block, token): 8 bsums as floats, d, padding
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+// 16-B runs a (quarters 0-1 or 2-3 of group lq & 1) to the lane's K quarter
+// of both groups: even gets group 0's 8 bytes, odd group 1's
+__device__ __forceinline__ void quarter_swap(const u32x4 a, u32x2& even, u32x2& odd) {
+  const auto s0 = __builtin_amdgcn_permlane16_swap(a.x, a.z, false, false);
+  const auto s1 = __builtin_amdgcn_permlane16_swap(a.y, a.w, false, false);
+  even = u32x2{s0[0], s1[0]};
+  odd = u32x2{s0[1], s1[1]};
+}
+__device__ __forceinline__ long pack_i64(u32x2 v) { return __builtin_bit_cast(long, v); }
+
+// The activation operands of block b: sub-block s of token lr % TP, TP = 16 /
+// NG, in the rows of group lr / TP and zero in the others' (xa[j] for group j)
+template <int NG>
+__device__ __forceinline__ void mt_load_x(const unsigned char* __restrict__ xq, int nb, int b,
+                                          int n_tokens, int lr, int lq, u32x2 (&xa)[NG][8]) {
+  constexpr int TP = 16 / NG;
+  const int t = min(lr % TP, n_tokens - 1);
+  const unsigned char* p = xq + (static_cast<long long>(t) * nb + b) * kQ8Bytes + 4 +
+                           32 * (lq & 1) + 16 * (lq >> 1);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    u32x2 e, o;
+    quarter_swap(*reinterpret_cast<const u32x4u*>(p + 64 * i), e, o);
+#pragma unroll
+    for (int j = 0; j < NG; ++j) {
+      const bool mine = NG == 1 || lr / TP == j;
+      xa[j][2 * i] = mine ? e : u32x2{0u, 0u};
+      xa[j][2 * i + 1] = mine ? o : u32x2{0u, 0u};
+    }
+  }
+}
+// d and the bsums (as floats) of every (block, token) into bst
+__device__ __forceinline__ void mt_stage_bs(const unsigned char* __restrict__ xq, int nb,
+                                            int n_tokens, float* bst, int tid, int nth) {
+  for (int i = tid; i < nb * n_tokens; i += nth) {  // i = block * n_tokens + token
+    const int b = i / n_tokens, t = i - b * n_tokens;
+    const uint32_t* p =
+        reinterpret_cast<const uint32_t*>(xq + (static_cast<long long>(t) * nb + b) * kQ8Bytes);
+    float* o = bst + i * kMtBsWords;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const uint32_t v = p[65 + s];
+      o[2 * s] = static_cast<float>(static_cast<int16_t>(v & 0xFFFFu));
+      o[2 * s + 1] = static_cast<float>(static_cast<int16_t>(v >> 16));
+    }
+    o[8] = __builtin_bit_cast(float, p[0]);
+  }
+}
+// ... of block b and the four tokens of the lane's results from it
+template <int TP>
+__device__ __forceinline__ void mt_load_bs(const float* bst, int b, int n_tokens, int lq,
+                                           float (&bs)[4][8], float (&xd)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int t = min((4 * lq) % TP + i, n_tokens - 1);
+    const float* p = bst + (b * n_tokens + t) * kMtBsWords;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) bs[i][s] = p[s];
+    xd[i] = p[8];
+  }
+}
+// The block sums of one result (NG row groups of one super-block): hd the
+// header of the lane's weight row, qw[j][g] its K quarter of group g's qs in
+// row group j.
+template <int NG>
+__device__ __forceinline__ void mt_block(const u32x4 hd, const u32x2 (&qw)[NG][4],
+                                         const u32x2 (&xa)[NG][8], const float (&bs)[4][8],
+                                         const float (&xd)[4], float (&sum)[4]) {
+  const ScaleMins sm8 = unpack_scales(hd.y, hd.z, hd.w);
+  const float d = half_bits_to_float(hd.x & 0xFFFFu);
+  const float dmin = half_bits_to_float(hd.x >> 16);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) sum[i] = 0.f;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    v4i ip = {0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < NG; ++j) {
+      const u32x2 q = (s & 1) ? qw[j][s >> 1] >> 4 : qw[j][s >> 1];
+      ip = __builtin_amdgcn_mfma_i32_16x16x32_i8(pack_i64(xa[j][s]), pack_i64(q & 0x0F0F0F0Fu), ip,
+                                                 0, 0, 0);
+    }
+    const float sd = d * byte_f(s < 4 ? sm8.sc_lo : sm8.sc_hi, s & 3);
+    const float smv = dmin * byte_f(s < 4 ? sm8.mn_lo : sm8.mn_hi, s & 3);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float t = __builtin_fmaf(sd, static_cast<float>(ip[i]), -(smv * bs[i][s]));
+      sum[i] = __builtin_fmaf(xd[i], t, sum[i]);
+    }
+  }
+}
+
+// Small matrices: a workgroup per 16 rows, loads straight into registers
+// (one memory latency before the arithmetic).  A lane loads the header of row
+// lr and two 16-B runs of its qs; a permlane16 swap turns two runs (quarters
+// 0-1 or 2-3 of two groups) into the lane's K quarter of each group.  With
+// more than 16 super-blocks per row a wave takes blocks w, w + 16, ... and the
+// row sums run on over these chunks.  Bound by latency.  Six tokens, cold in a
+// graph, against a wave per row group that looped over the tokens with sdot4:
+// 8192 x 2048 11.8 -> 6.1 us, 2048 x 4096 17.8 -> 6.5, 64 x 2048 9.0 -> 3.8.
+constexpr int kMtWaves = 16;
+template <bool kChunked, typename Out>
+__global__ void __launch_bounds__(64 * kMtWaves) gemv_mt_kernel(
+    const sg_block_q4k* __restrict__ w, const unsigned char* __restrict__ xq, Out y, int n_rows,
+    int nb, int n_tokens) {
+  extern __shared__ __attribute__((aligned(16))) float mt_lds[];  // [2][waves][256], then bs
+  const int tid = threadIdx.x, nth = blockDim.x, lane = tid & 63, wave = tid >> 6;
+  const int nwv = nth >> 6;  // min(nb, kMtWaves)
+  const int lr = lane & 15, lq = lane >> 4;
+  float* bst = mt_lds + 2 * nwv * 256;
+  const int n_chunks = kChunked ? (nb + nwv - 1) / nwv : 1;
+  const int row0 = blockIdx.x * 16;
+  const sg_block_q4k* wr = w + static_cast<long long>(min(row0 + lr, n_rows - 1)) * nb;
+  u32x4 hd, q0, q1;
+  auto load_w = [&](int b) {
+    const char* p = reinterpret_cast<const char*>(wr + b);
+    hd = *reinterpret_cast<const u32x4u*>(p);
+    p += 16 + 32 * (lq & 1) + 16 * (lq >> 1);
+    q0 = *reinterpret_cast<const u32x4u*>(p);
+    q1 = *reinterpret_cast<const u32x4u*>(p + 64);
+  };
+  u32x2 xa[1][8];
+  load_w(wave);  // (wave < nwv <= nb)
+  mt_load_x<1>(xq, nb, wave, n_tokens, lr, lq, xa);
+  mt_stage_bs(xq, nb, n_tokens, bst, tid, nth);
+  bar();
+  float run = 0.f;  // of output tid: token 4 (tid >> 4 & 3) + (tid >> 6), row tid & 15
+  for (int c = 0; c < n_chunks; ++c) {
+    const int b = c * nwv + wave;
+    float* part = mt_lds + (c & 1) * nwv * 256;
+    if (!kChunked || b < nb) {
+      u32x2 qw[1][4];
+      quarter_swap(q0, qw[0][0], qw[0][1]);
+      quarter_swap(q1, qw[0][2], qw[0][3]);
+      float bs[4][8], xd[4], sum[4];
+      mt_load_bs<16>(bst, b, n_tokens, lq, bs, xd);
+      mt_block<1>(hd, qw, xa, bs, xd, sum);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) part[wave * 256 + 64 * i + lane] = sum[i];
+      if (kChunked && b + nwv < nb) {
+        load_w(b + nwv);
+        mt_load_x<1>(xq, nb, b + nwv, n_tokens, lr, lq, xa);
+      }
+    }
+    bar();  // (the other buffer is free again: its readers passed this barrier too)
+    const int nbc = min(nwv, nb - c * nwv);
+    if (nth >= 256) {
+      if (tid < 256)
+        for (int i = 0; i < nbc; ++i) run += part[i * 256 + tid];
+    } else {  // fewer than four waves (one chunk): several outputs per thread
+      for (int v = tid; v < 256; v += nth) {
+        float acc = 0.f;
+        for (int i = 0; i < nbc; ++i) acc += part[i * 256 + v];
+        const int t = 4 * ((v >> 4) & 3) + (v >> 6), r = row0 + (v & 15);
+        if (t < n_tokens && r < n_rows) y.store(t * n_rows + r, acc);
+      }
+    }
+  }
+  if (nth >= 256 && tid < 256) {
+    const int t = 4 * ((tid >> 4) & 3) + (tid >> 6), r = row0 + (tid & 15);
+    if (t < n_tokens && r < n_rows) y.store(t * n_rows + r, run);
+  }
+}
+
+// Large matrices: persistent workgroups take sets of 16 RG rows in turn.
+// The rows stream through a ring of three LDS buffers (two sets in flight)
+// with buffer_load ... lds in 1-KB instructions; one barrier per set: set
+// i's copies have landed, set i - 1's block sums are complete and its buffer
+// and set i - 2's sums are free.  A row is an odd number of 16-B chunks (nb *
+// 9, and one of padding where that is even), so that the 16 rows a wave reads
+// together start in different banks.
+//
+// With up to 8 tokens a 16 x 16 result would be half padding, and its
+// epilogue, four operations per result and sub-block, is most of what the
+// kernel issues.  NG = 2 row groups then share a result: group j's tokens sit
+// in rows 8j..8j+7 of its A operand, zero elsewhere, and the two groups' MFMAs
+// accumulate into one result whose row half j is group j's.
+//
+// Bound by the weight stream: 248320 x 2048 x 4 tokens 77.6 -> 54.8 us (5.3
+// TB/s).  With 64-row sets loaded straight to registers it took 70 us: 16-B
+// pieces of a 128-B line asked for by several instructions, against whole
+// lines here.
+constexpr int kMtwBufs = 3;
+constexpr int kMtwCopies = 5;  // copy instructions per wave and set, at most
+__host__ __device__ constexpr int mtw_buf_words(int rg, int nb) {
+  return (16 * rg * (9 * nb | 1) + 63) / 64 * 256;
+}
+
+template <int NG, int RG, int kMaxWv, typename Out>
+__global__ void __launch_bounds__(64 * kMaxWv) gemv_mtw_kernel(
+    const sg_block_q4k* __restrict__ w, const unsigned char* __restrict__ xq, Out y, int n_rows,
+    int nb, int n_tokens) {
+  constexpr int TP = 16 / NG;       // token rows of one row group in a result
+  constexpr int kSets = RG / NG;    // results (of 4 registers) per super-block, a wave each
+  constexpr int kOuts = kSets * 256;  // outputs of a set, tokens past n_tokens included
+  extern __shared__ __attribute__((aligned(16))) uint32_t mtw_lds[];
+  const int tid = threadIdx.x, nth = blockDim.x, lane = tid & 63, wave = tid >> 6;
+  const int nwv = nth >> 6;  // = nb * kSets
+  const int ws = kSets == 1 ? 0 : wave / nb, wb = wave - ws * nb;  // the wave's result, block
+  const int lr = lane & 15, lq = lane >> 4;
+  const int cpr = 9 * nb | 1, rw = 4 * cpr;  // chunks and words of a row in LDS
+  const int bufw = mtw_buf_words(RG, nb);
+  uint32_t* ring = mtw_lds;
+  float* part = reinterpret_cast<float*>(ring + kMtwBufs * bufw);  // [2][nwv][256]
+  float* bst = part + 2 * nwv * 256;
+  const int n_sets = (n_rows + 16 * RG - 1) / (16 * RG);
+  const uint32_t row_bytes = nb * kQ4Bytes;
+
+  // copy instruction wave + nwv i of a set: its lane's chunk, from the set's
+  // first row (the padding chunk re-reads the row's first)
+  const int n_inst = bufw / 256;
+  uint32_t ofs[kMtwCopies];
+#pragma unroll
+  for (int i = 0; i < kMtwCopies; ++i) {
+    const int c = min((wave + nwv * i) * 64 + lane, 16 * RG * cpr - 1);
+    const int r = c / cpr, p = c - r * cpr;
+    ofs[i] = r * row_bytes + (p == 9 * nb ? 0 : 16 * p);
+  }
+  const int mine = (n_inst - wave + nwv - 1) / nwv;  // this wave's instructions per set
+  auto issue = [&](int g, int slot) {
+    const long long r0 = static_cast<long long>(g) * 16 * RG;
+    const int rows = min(16 * RG, static_cast<int>(n_rows - r0));
+    // rows past the matrix are out of the buffer's range and read as zero
+    const u32x4 rs = buffer_desc(reinterpret_cast<const char*>(w) + r0 * row_bytes,
+                                 rows * row_bytes);
+#pragma unroll
+    for (int i = 0; i < kMtwCopies; ++i)
+      if (i < mine) dma16<true>(ring + slot * bufw + 256 * (wave + nwv * i), ofs[i], rs, 0);
+  };
+  const int g0 = blockIdx.x, gs = gridDim.x;
+  if (g0 < n_sets) issue(g0, 0);
+  if (g0 + gs < n_sets) issue(g0 + gs, 1);
+  u32x2 xa[NG][8];
+  float bs[4][8], xd[4];
+  mt_load_x<NG>(xq, nb, wb, n_tokens, lr, lq, xa);
+  mt_stage_bs(xq, nb, n_tokens, bst, tid, nth);
+  bar();
+  mt_load_bs<TP>(bst, wb, n_tokens, lq, bs, xd);
+
+  auto finish = [&](int g, const float* pr) {  // add the block sums of set g and store
+    for (int v = tid; v < kOuts; v += nth) {
+      float acc = 0.f;
+      const int vm = v >> 8;
+      for (int i = 0; i < nb; ++i) acc += pr[(vm * nb + i) * 256 + (v & 255)];
+      const int vi = (v >> 6) & 3, vq = (v >> 4) & 3;
+      const int t = (4 * vq) % TP + vi;
+      const int r = (g * RG + vm * NG + vq * NG / 4) * 16 + (v & 15);
+      if (t < n_tokens && r < n_rows) y.store(t * n_rows + r, acc);
+    }
+  };
+  int slot = 0, buf = 0;
+  for (int g = g0; g < n_sets; g += gs) {
+    // the oldest set has landed once only the next one's copies are left
+    wait_vm_n(g + gs < n_sets ? mine : 0);
+    bar();
+    const int s2 = slot == 0 ? 2 : slot - 1;  // (slot + 2) % 3
+    if (g + 2 * gs < n_sets) issue(g + 2 * gs, s2);
+    if (g != g0) finish(g - gs, part + (buf ^ 1) * nwv * 256);
+    const uint32_t* rb = ring + slot * bufw + 36 * wb + ws * NG * 16 * rw;
+    const u32x4 hd = *reinterpret_cast<const u32x4*>(rb + (lq * NG / 4 * 16 + lr) * rw);
+    u32x2 qw[NG][4];
+#pragma unroll
+    for (int j = 0; j < NG; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        qw[j][q] = *reinterpret_cast<const u32x2*>(rb + (j * 16 + lr) * rw + 4 + 8 * q + 2 * lq);
+    float sum[4];
+    mt_block<NG>(hd, qw, xa, bs, xd, sum);
+    float* pw = part + (buf * nwv + wave) * 256;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) pw[64 * i + lane] = sum[i];
+    slot = slot == 2 ? 0 : slot + 1;
+    buf ^= 1;
+  }
+  bar();
+  if (g0 < n_sets)
+    finish(g0 + (n_sets - 1 - g0) / gs * gs, part + (buf ^ 1) * nwv * 256);
 }
 
 // dots[(r*nb + b)*8 + s] = int32 sub-block dot (test hook).
@@ -467,6 +764,14 @@ static int check_gemv_geometry(const char* name, int n_rows, int k) {
   return SG_OK;
 }
 
+// LDS of a gemv1 launch (the staged activations and the waves' results)
+constexpr size_t kGemv1MaxLds = 96 * 1024;
+static size_t gemv1_lds(int n_rows, int nb) {
+  const int rpw = 64 / lanes_per_row(nb);
+  return static_cast<size_t>(nb) * kXStride * 4 +
+         gemv1_launch((static_cast<long long>(n_rows) + rpw - 1) / rpw, rpw).res_bytes;
+}
+
 // one gemv1 launch over a row source and an output policy (shared by the
 // fp16-output entry points)
 template <typename Rows, typename Out>
@@ -477,7 +782,7 @@ static int launch_gemv1(Rows rows, const sg_block_q8k* x, Out out, int n_rows, i
   const long long n_groups = (n_rows + (64 / lpr) - 1) / (64 / lpr);
   const Gemv1Launch L = gemv1_launch(n_groups, 64 / lpr);
   const size_t lds = static_cast<size_t>(nb) * kXStride * 4 + L.res_bytes;
-  if (lds > 96 * 1024)
+  if (lds > kGemv1MaxLds)
     return set_error(SG_ERR_UNSUPPORTED, "%s: n_rows=%d k=%d needs %zu B of LDS", nm, n_rows, k,
                      lds);
   gemv1_go(L, lds, s, rows, x, out, n_rows, nb, lpr);
@@ -508,6 +813,55 @@ static int launch_ptrs(const sg_block_q4k* const* ptrs, const sg_block_q8k* x, O
   return check_launch(nm);
 }
 
+// Which several-token kernel, by super-blocks (n_rows * nb), measured cold in
+// graphs (us, quantizer included):
+// - gemv_batched_kernel: at most eight staged blocks of two to four tokens in
+//   a matrix of 65536 or more (262141 x 512: 2 tokens 17.8 against 20.4 for
+//   the streaming kernel; 3 tokens 19.7 / 20.6; 4 tokens x 1024 23.1 / 20.3);
+// - gemv_mtw_kernel, the streaming one: from 131072 with more than 8 blocks
+//   per row (8197 x 4096: 11.5 against 13.7; 4096 x 4096: 8.3 / 7.4), from
+//   262144 below that (32765 x 2048: 12.9 / 15.2; 16381 x 2048: 10.0 / 10.0); with
+//   more than 8 tokens, whose sets are twice the work, from 524288 (65533 x
+//   2048: 23.7 / 26.0; 32765: 15.8 / 15.7) and only with more than 4 blocks
+//   per row (131069 x 1024: 25.8 / 22.6);
+// - gemv_mt_kernel otherwise.
+static bool use_batched_sdot(int n_rows, int nb, int n_tokens) {
+  return n_tokens >= 2 && n_tokens <= 4 && n_tokens * nb <= 8 &&
+         static_cast<long long>(n_rows) * nb >= 65536;
+}
+static bool use_mtw(int n_rows, int nb, int n_tokens) {
+  if (nb < 2 || nb > 16 || (n_tokens > 8 && nb <= 4)) return false;
+  return static_cast<long long>(n_rows) * nb >=
+         (nb > 8 ? 131072 : (n_tokens <= 8 ? 262144 : 524288));
+}
+
+template <int NG, int RG, int kMaxWv, typename Out>
+static void gemv_mtw_go(hipStream_t s, const sg_block_q4k* w, const unsigned char* xb, Out y,
+                        int n_rows, int nb, int n_tokens) {
+  const int n_sets = (n_rows + 16 * RG - 1) / (16 * RG);
+  const size_t lds = (static_cast<size_t>(kMtwBufs) * mtw_buf_words(RG, nb) +
+                      2 * static_cast<size_t>(nb) * (RG / NG) * 256 +
+                      static_cast<size_t>(nb) * n_tokens * kMtBsWords) * 4;
+  const int per_cu = std::min<int>(160 * 1024 / lds, 32 / (nb * (RG / NG)));  // resident workgroups
+  const int cap = 256 * per_cu;
+  hipLaunchKernelGGL((gemv_mtw_kernel<NG, RG, kMaxWv, Out>), dim3(n_sets < cap ? n_sets : cap),
+                     dim3(64 * nb * (RG / NG)), lds, s, w, xb, y, n_rows, nb, n_tokens);
+}
+template <typename Out>
+static void gemv_mt_go(hipStream_t s, const sg_block_q4k* w, const unsigned char* xb, Out y,
+                       int n_rows, int nb, int n_tokens) {
+  const int nwv = nb < kMtWaves ? nb : kMtWaves;
+  const size_t lds = (2 * static_cast<size_t>(nwv) * 256 +
+                      static_cast<size_t>(nb) * n_tokens * kMtBsWords) * 4;
+  const dim3 grid((n_rows + 15) / 16), block(64 * nwv);
+  if (nb <= kMtWaves)
+    hipLaunchKernelGGL((gemv_mt_kernel<false, Out>), grid, block, lds, s, w, xb, y, n_rows, nb,
+                       n_tokens);
+  else
+    hipLaunchKernelGGL((gemv_mt_kernel<true, Out>), grid, block, lds, s, w, xb, y, n_rows, nb,
+                       n_tokens);
+}
+
 // the batched GEMV over an output policy (fp32 or fp16 rows)
 template <typename Out>
 static int launch_batched(const sg_block_q4k* w, const sg_block_q8k* x, Out y, int n_rows, int k,
@@ -519,13 +873,29 @@ static int launch_batched(const sg_block_q4k* w, const sg_block_q8k* x, Out y, i
                      kMaxTokens);
   if (static_cast<long long>(n_rows) * n_tokens > 0x7fffffffLL)
     return set_error(SG_ERR_GEOMETRY, "%s: n_rows*n_tokens too large", nm);
-  const int nb = k / kQK, lpr = lanes_per_row(nb);
-  const size_t lds = static_cast<size_t>(nb) * n_tokens * kXStride * 4;
-  if (lds > 96 * 1024)
+  const int nb = k / kQK;
+  if (static_cast<size_t>(nb) * n_tokens * kXStride * 4 > 96 * 1024)
     return set_error(SG_ERR_UNSUPPORTED, "%s: k*n_tokens too large for LDS", nm);
-  const long long n_groups = (n_rows + (64 / lpr) - 1) / (64 / lpr);
-  hipLaunchKernelGGL((gemv_batched_kernel<Out>), dim3(gemv_grid(n_groups)), dim3(256), lds, s, w,
-                     reinterpret_cast<const unsigned char*>(x), y, n_rows, nb, lpr, n_tokens);
+  const unsigned char* xb = reinterpret_cast<const unsigned char*>(x);
+  if (n_tokens == 1) {  // the one-token GEMV, where its results fit LDS
+    if (gemv1_lds(n_rows, nb) <= kGemv1MaxLds)
+      return launch_gemv1(PlainRows{w, nb}, x, y, n_rows, k, s, nm);
+  }
+  if (use_batched_sdot(n_rows, nb, n_tokens)) {
+    const int lpr = lanes_per_row(nb);
+    const long long n_groups = (n_rows + (64 / lpr) - 1) / (64 / lpr);
+    hipLaunchKernelGGL((gemv_batched_kernel<Out>), dim3(gemv_grid(n_groups)), dim3(256),
+                       static_cast<size_t>(nb) * n_tokens * kXStride * 4, s, w, xb, y, n_rows, nb,
+                       lpr, n_tokens);
+  } else if (!use_mtw(n_rows, nb, n_tokens)) {
+    gemv_mt_go(s, w, xb, y, n_rows, nb, n_tokens);
+  } else if (nb > 8) {
+    gemv_mtw_go<1, 1, 16>(s, w, xb, y, n_rows, nb, n_tokens);
+  } else if (n_tokens <= 8) {
+    gemv_mtw_go<2, 2, 8>(s, w, xb, y, n_rows, nb, n_tokens);
+  } else {
+    gemv_mtw_go<1, 2, 16>(s, w, xb, y, n_rows, nb, n_tokens);
+  }
   return check_launch(nm);
 }
 

@@ -6,6 +6,8 @@
 // shared-expert sigmoid gate (norm_rotary.cu:177-184, moe.cu:282-292) and
 // the fp32 x fp16 GEMV that produces gate and router logits
 // (q4_k.cu:133-149, 285-303).
+#include <type_traits>
+
 #include "sg_common.hpp"
 #include "sg_router.hpp"
 
@@ -107,21 +109,193 @@ __global__ void __launch_bounds__(256) sigmoid_gate_f16_kernel(uint16_t* __restr
   out[r * hidden + i] = f16b(f16v(out[r * hidden + i]) * s);
 }
 
-// y[t][r] = W[r] . f32(x[t]) with W fp32 [n_rows][k], x fp16 [T][k]: eight
-// rows per workgroup, one per 32-lane half-wave, in the reference's lane
-// order (rowdot_f32_lanes32).
-__global__ void __launch_bounds__(256) gemv_f32_f16x_kernel(const float* __restrict__ w,
-                                                            const uint16_t* __restrict__ x,
-                                                            float* __restrict__ y, int n_rows,
-                                                            int k) {
+// y[t][r] = W[r] . f32(x[t]) with W fp32 [n_rows][k], x fp16 [T][k]: two
+// rows per one-wave workgroup, one per 32-lane half, in the reference's lane
+// order (rowdot_f32_lanes32).  One wave per workgroup spreads a router's 256
+// rows over 128 CUs.
+__global__ void __launch_bounds__(64) gemv_f32_f16x_kernel(const float* __restrict__ w,
+                                                           const uint16_t* __restrict__ x,
+                                                           float* __restrict__ y, int n_rows,
+                                                           int k) {
   const int l = threadIdx.x & 31;
-  const int row = blockIdx.x * 8 + (threadIdx.x >> 5);
+  const int row = blockIdx.x * 2 + (threadIdx.x >> 5);
   const long long t = blockIdx.y;
   const int r = row < n_rows ? row : n_rows - 1;  // whole halves stay active for the shuffles
   const uint16_t* xt = x + t * k;
   const float v = rowdot_f32_lanes32(w + static_cast<long long>(r) * k,
                                      [&](int i) { return f16v(xt[i]); }, k, l);
   if (l == 0 && row < n_rows) y[t * n_rows + row] = v;
+}
+
+// The same for many tokens (a prefill chunk's router logits) on the fp32
+// matrix cores, bit for bit: v_mfma_f32_16x16x1_4b_f32 is four independent
+// 16 x 16 outer products, K = 1, each element one fused multiply-add.  The
+// reference order's 32 lane sums of an output (elements l, l + 32, ...) are 32
+// chains that never meet before the final tree, so each is a block of an
+// accumulator of its own: eight MFMAs of four blocks (b) per 32 elements.  Two
+// waves share a tile of 16 rows x 16 tokens: wave h takes lane sums 16 h ..
+// 16 h + 15 (four MFMAs, m), lane 16 b + i reading sums 16 h + 4 b .. + 3 of row
+// i (16 B) and token i (8 B), and holds those 16 sums of its four outputs; the
+// tree's first level (offset 16) meets the other wave's through LDS.
+//
+// A workgroup is WR x WT tiles.  W and x stream through a ring of LDS buffers,
+// kRgK elements of every row at a time; chunk c of row r lies at c ^ (r & 15), so
+// that the sixteen rows of a read start in different banks.  A step's operands
+// are read while the previous one multiplies, over the slots' barriers too.
+// What bounds it is the matrix core: one of these MFMAs takes 64 cycles, the
+// vector ALU's rate.  2048 tokens x 256 rows x k 2048: 229 -> 29.0 us (74
+// TFLOP/s), where a half-wave per output re-read 12 KB for each.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+constexpr int kRgK = 128;    // elements per ring slot: 32 chunks of a W row, 16 of an x row
+template <int WR, int WT, int Ring>
+struct RgTile {
+  static constexpr int ring = Ring;
+  static constexpr int rows = 16 * WR, toks = 16 * WT, waves = 2 * WR * WT;
+  static constexpr int w_inst = rows * 32 / 64, x_inst = toks * 16 / 64;  // 1-KB copies per slot
+  static constexpr int n_inst = w_inst + x_inst;
+  static_assert(n_inst % waves == 0, "every wave issues the same number of copies");
+  static constexpr int mine = n_inst / waves;
+  static constexpr int slot_words = n_inst * 256;
+  static constexpr size_t lds = static_cast<size_t>(ring) * slot_words * 4;
+  static_assert(lds >= waves * 8192, "the final exchange fits the ring");
+};
+// The tiles' time is their chain, k / 32 steps of four MFMAs (11.4 us at k =
+// 2048 however few tiles), the row-per-half-wave kernel's grows with the
+// outputs: 256 x 2048 at 57 tokens 8.6 us against 11.4 for the tiles, at 128
+// tokens 16.6 / 11.5, 60 x 1280 at 64 tokens 3.4 / 8.2, at 509 11.6 / 8.4.
+// Tiles of 32 x 32 read a third less through L2 and win once they fill
+// the chip (256 x 2048 at 509 tokens 15.6 against 11.7 us for 16 x 32, at 1024
+// 16.9 / 17.1, at 2048 29.0 / 31.5).
+constexpr long long kTileOutputs = 96 * 256, kBigTileOutputs = 1024 * 256;
+
+template <int WR, int WT, int kRgRing>
+__global__ void __launch_bounds__(128 * WR * WT) gemv_f32_f16x_tile_kernel(
+    const float* __restrict__ w, const uint16_t* __restrict__ x, float* __restrict__ y, int n_rows,
+    int k, int n_tokens, int n_rt) {
+  using Tile = RgTile<WR, WT, kRgRing>;
+  extern __shared__ __attribute__((aligned(16))) uint32_t rg_lds[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r0 = blockIdx.x % n_rt * Tile::rows, t0 = blockIdx.x / n_rt * Tile::toks;
+  const int h = __builtin_amdgcn_readfirstlane(wave & 1), tile = wave >> 1, wr = tile % WR, wt = tile / WR;
+  const int i = lane & 15, b = lane >> 4;
+
+  // the wave's copies of a slot: instruction wave + waves j; LDS chunk q of
+  // the W part is chunk (q % 32) ^ (row & 15) of row q / 32, of the x part
+  // chunk (q % 16) ^ (t & 15) of token q / 16 (rows and tokens past the end
+  // repeat the last)
+  const u32x4 rw = buffer_desc(w, static_cast<uint32_t>(n_rows) * k * 4u);
+  const u32x4 rx = buffer_desc(x, static_cast<uint32_t>(n_tokens) * k * 2u);
+  uint32_t ofs[Tile::mine];
+#pragma unroll
+  for (int j = 0; j < Tile::mine; ++j) {
+    const int inst = wave + Tile::waves * j;
+    if (inst < Tile::w_inst) {
+      const int q = inst * 64 + lane, r = q >> 5, c = (q & 31) ^ (r & 15);
+      ofs[j] = static_cast<uint32_t>(min(r0 + r, n_rows - 1)) * k * 4u + 16 * c;
+    } else {
+      const int q = (inst - Tile::w_inst) * 64 + lane, t = q >> 4, c = (q & 15) ^ (t & 15);
+      ofs[j] = static_cast<uint32_t>(min(t0 + t, n_tokens - 1)) * k * 2u + 16 * c;
+    }
+  }
+  auto issue = [&](int c, int slot) {  // elements kRgK c .. into ring slot `slot`
+#pragma unroll
+    for (int j = 0; j < Tile::mine; ++j) {
+      const int inst = wave + Tile::waves * j;
+      uint32_t* dst = rg_lds + slot * Tile::slot_words + 256 * inst;
+      if (inst < Tile::w_inst) dma16(dst, ofs[j], rw, c * kRgK * 4);
+      else dma16(dst, ofs[j], rx, c * kRgK * 2);
+    }
+  };
+  const int n_c = k / kRgK;
+#pragma unroll
+  for (int c = 0; c < kRgRing - 1; ++c)
+    if (c < n_c) issue(c, c);
+
+  f32x16 acc[4] = {};
+  f32x4 av[2];
+  uint2 hv[2];
+  // Slot c has landed once only the next slots' copies are left (at the end:
+  // none); after the barrier every wave's have, and slot c - 1 is free.
+  int slot = 0, free = kRgRing - 1;  // of the chunk being read, of the next to issue
+  auto enter = [&](int c) {
+    wait_vm_sets<1, (kRgRing - 2) * Tile::mine>(c + kRgRing - 2 < n_c);
+    bar();
+    if (c + kRgRing - 1 < n_c) issue(c + kRgRing - 1, free);
+    free = free + 1 == kRgRing ? 0 : free + 1;
+  };
+  // the lane's word of W and x in a slot at step j (chunk 8 j + 4 h + b and 4 j
+  // + 2 h + b / 2 of its rows, placed as above)
+  int aw[kRgK / 32], ax[kRgK / 32];
+#pragma unroll
+  for (int j = 0; j < kRgK / 32; ++j) {
+    aw[j] = (16 * wr + i) * 128 + 4 * ((8 * j + 4 * h + b) ^ i);
+    ax[j] = Tile::w_inst * 256 + (16 * wt + i) * 64 + 4 * ((4 * j + 2 * h + (b >> 1)) ^ i) +
+            2 * (b & 1);
+  }
+  auto read = [&](int j, int o) {  // step j of the slot into operand set o
+    const uint32_t* s = rg_lds + slot * Tile::slot_words;
+    av[o] = *reinterpret_cast<const f32x4*>(s + aw[j]);
+    hv[o] = *reinterpret_cast<const uint2*>(s + ax[j]);
+  };
+  enter(0);
+  read(0, 0);
+  for (int c = 0; c < n_c; ++c) {
+#pragma unroll
+    for (int j = 0; j < kRgK / 32; ++j) {
+      const int o = j & 1;
+      // the next step's reads stay in front of this one's MFMAs (the
+      // compiler would move them down to their use and wait there)
+      const float bv[4] = {f16v(hv[o].x & 0xFFFFu), f16v(hv[o].x >> 16), f16v(hv[o].y & 0xFFFFu),
+                           f16v(hv[o].y >> 16)};
+      if (j + 1 < kRgK / 32) {
+        read(j + 1, o ^ 1);
+      } else if (c + 1 < n_c) {
+        enter(c + 1);
+        slot = slot + 1 == kRgRing ? 0 : slot + 1;
+        read(0, o ^ 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        acc[m] = __builtin_amdgcn_mfma_f32_16x16x1f32(av[o][m], bv[m], acc[m], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  // Lane sum 16 h + 4 q + m of the lane's output r (row 4 b + r, token i) is
+  // element 4 q + r of acc[m]; the tree adds at offsets 16, 8, 4, 2, 1.  Wave
+  // h gives the other its sums of outputs 2 (1 - h), 2 (1 - h) + 1 and finishes
+  // outputs 2 h, 2 h + 1 (the sum of two is the same in either order).
+  bar();  // the ring is free
+  float* ex = reinterpret_cast<float*>(rg_lds) + 2048 * wave + lane;  // [32][64] per wave
+  const float* ox = reinterpret_cast<const float*>(rg_lds) + 2048 * (wave ^ 1) + lane;
+  const int t = t0 + 16 * wt + i;
+  auto finish = [&](auto hc) {
+    constexpr int H = decltype(hc)::value;
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) ex[64 * (8 * m + 2 * q + u)] = acc[m][4 * q + 2 * (1 - H) + u];
+    bar();
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      float v[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        float s[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s[q] = acc[m][4 * q + 2 * H + u] + ox[64 * (8 * m + 2 * q + u)];
+        v[m] = (s[0] + s[2]) + (s[1] + s[3]);
+      }
+      const int row = r0 + 16 * wr + 4 * b + 2 * H + u;
+      if (row < n_rows && t < n_tokens)
+        y[static_cast<long long>(t) * n_rows + row] = (v[0] + v[2]) + (v[1] + v[3]);
+    }
+  };
+  if (h) finish(std::integral_constant<int, 1>{});
+  else finish(std::integral_constant<int, 0>{});
 }
 
 // Router GEMV and top-k of one token in one launch (mmq.cu:459-511): the
@@ -281,8 +455,28 @@ int sg_gemv_f32_out_f16x(const float* w, const uint16_t* x, float* y, int n_rows
   if (n_rows <= 0 || k <= 0 || n_tokens <= 0 || n_tokens > 65535)
     return set_error(SG_ERR_GEOMETRY, "sg_gemv_f32_out_f16x: n_rows=%d k=%d n_tokens=%d", n_rows,
                      k, n_tokens);
-  hipLaunchKernelGGL(gemv_f32_f16x_kernel, dim3((n_rows + 7) / 8, n_tokens), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), w, x, y, n_rows, k);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  // The tiles copy 16-B chunks of whole kRgK-element runs through 32-bit buffer
+  // offsets
+  const long long outs = static_cast<long long>(n_rows) * n_tokens;
+  const bool tiles = k % kRgK == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
+                     reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+                     static_cast<long long>(n_rows) * k * 4 < 0x80000000LL &&
+                     static_cast<long long>(n_tokens) * k * 2 < 0x80000000LL;
+  auto tiled = [&](auto tile, auto kern) {
+    using Tile = decltype(tile);
+    const int n_rt = (n_rows + Tile::rows - 1) / Tile::rows;
+    const int n_tt = (n_tokens + Tile::toks - 1) / Tile::toks;
+    hipLaunchKernelGGL(kern, dim3(n_rt * n_tt), dim3(64 * Tile::waves), Tile::lds, s, w, x, y,
+                       n_rows, k, n_tokens, n_rt);
+  };
+  if (tiles && outs >= kBigTileOutputs)
+    tiled(RgTile<2, 2, 3>{}, gemv_f32_f16x_tile_kernel<2, 2, 3>);
+  else if (tiles && outs >= kTileOutputs)
+    tiled(RgTile<1, 2, 5>{}, gemv_f32_f16x_tile_kernel<1, 2, 5>);
+  else
+    hipLaunchKernelGGL(gemv_f32_f16x_kernel, dim3((n_rows + 1) / 2, n_tokens), dim3(64), 0, s, w, x,
+                       y, n_rows, k);
   return check_launch("sg_gemv_f32_out_f16x");
 }
 

@@ -170,6 +170,17 @@ __device__ __forceinline__ void dma16(const uint32_t* lds, uint32_t voff, u32x4 
                  : "memory");
 }
 
+// The same from a per-lane global address (non-temporal; lanes off are not
+// written), for copies that run beside LDS reads.
+__device__ __forceinline__ void dma16_stream(const uint32_t* lds, const char* src) {
+  const uint32_t l =
+      __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds)));
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt"
+               :
+               : "s"(l), "v"(src)
+               : "memory");
+}
+
 // a pointer the caller knows to be wave-uniform, moved to scalar registers
 template <typename T>
 __device__ __forceinline__ T* uniform_ptr(T* p) {

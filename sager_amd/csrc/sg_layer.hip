@@ -1,6 +1,7 @@
 // sg_layer.hip - one fused MoE layer (decode step or verify window) on gfx950.
 //
-// Two launches per layer, on one stream:
+// Two launches per layer of one token, on one stream (several tokens: the
+// routing launch, the gate/up launch, with many the Q8_K of h, then back):
 //
 //   front  grid (row chunks of 16, groups + 1): every routed workgroup finds
 //          its expert from the top-k by logit, starts streaming that
@@ -17,8 +18,8 @@
 //
 // Weights stream from HBM into LDS with global_load_lds_dwordx4 (1 KB of
 // consecutive memory per instruction) and are read back per lane at the
-// 144-B super-block stride.  A group is the shared expert (group 0, tokens
-// 0..T-1 in slot k) or one distinct routed expert (ascending id) with its
+// 144-B super-block stride.  A group is the shared expert (the first groups:
+// tokens in slot k, a few per group) or one distinct routed expert (ascending id) with its
 // (token, slot) routes; an expert shared by several tokens is streamed once.
 // Loads that do not depend on routing (x, h, residual) are issued at kernel
 // start so their latency overlaps the routing and the plan load.
@@ -37,7 +38,6 @@ namespace sg {
 constexpr int kLMaxExperts = 1024;
 constexpr int kLMaxK = 32;
 constexpr int kLMaxTokens = 16;
-constexpr int kMaxEpt = 16;        // experts per routing thread (1-wave teams, E = 1024)
 
 __host__ __device__ constexpr inline int pow2_ceil(int n) {
   int l = 1;
@@ -50,7 +50,6 @@ __host__ __device__ constexpr inline int pow2_ceil(int n) {
 struct LayerPlan {
   int* meta;    // [0] groups, [1] has_shared, [2] valid routes
   int* off;     // [gmax+1] entry offsets per group
-  int* expert;  // [gmax] expert id per group, -1 = shared expert
   int* tok;     // [emax] entry token
   int* slot;    // [emax] entry slot
   unsigned long long* wdown;  // [gmax] down matrix of the group, 0 = absent expert
@@ -59,20 +58,20 @@ struct LayerPlan {
 };
 
 struct LayerWs {
-  size_t meta, off, expert, tok, slot, wdown, wgate, wup, sgate, h, xq, total;
+  size_t meta, off, tok, slot, wdown, wgate, wup, sgate, h, xq, total;
   int gmax, emax;
 };
 
 static size_t align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
-static LayerWs layer_ws(int T, int hidden, int n_ff, int E, int k) {
+// split: tokens per group of the shared expert (several tokens; see kShSplit)
+static LayerWs layer_ws(int T, int hidden, int n_ff, int E, int k, int split) {
   LayerWs w{};
-  w.gmax = (T * k < E ? T * k : E) + 1;
+  w.gmax = (T * k < E ? T * k : E) + (T + split - 1) / split;
   w.emax = T * k + T;
   size_t o = 0;
   w.meta = o;   o = align256(o + 4 * sizeof(int));
   w.off = o;    o = align256(o + (w.gmax + 1) * sizeof(int));
-  w.expert = o; o = align256(o + w.gmax * sizeof(int));
   w.tok = o;    o = align256(o + w.emax * sizeof(int));
   w.slot = o;   o = align256(o + w.emax * sizeof(int));
   w.wdown = o;  o = align256(o + w.gmax * sizeof(unsigned long long));
@@ -88,9 +87,9 @@ static LayerWs layer_ws(int T, int hidden, int n_ff, int E, int k) {
 }
 
 struct FrontLds {
-  int nteams, tw, TT, ept, m, e32, ncp;
-  int tabg, tabu, tabd, lv, ev, cand, top, red, zs, spec, ridx, rw, re, rfirst, poff, pexp,
-      ptok, pslot, ctrl, kw, xs, total;
+  int ept, m, e32, ncp;
+  int tabg, tabu, tabd, lv, ev, cand, top, red, zs, ridx, rw, re, rfirst, poff, pexp, ptok, pslot,
+      ctrl, kw, xs, total;
 };
 
 struct LayerArgs {
@@ -115,7 +114,8 @@ struct LayerArgs {
   float shared_w;
   int back_rows, back_lrow;  // rows per back workgroup, lanes per row there
   int back_bufs;             // back waves with a down-row buffer (8, or 4 when LDS is short)
-  int publish_only;          // front launch of the publisher alone (the routing launch)
+  int split;                 // tokens per group of the shared expert
+  int hq_pre;                // h is quantized (in place) before the back launch
   FrontLds front_routed, front_shared;  // front LDS layouts (routing groups, shared group)
   // the session's fp16 buffers (after the fields above, whose layout the
   // fp32 kernels read): fp16 x16 instead of x, or (with either, or alone
@@ -128,20 +128,16 @@ struct LayerArgs {
   uint16_t* out16;
 };
 
-// ---- front kernel LDS layout (dwords) -----------------------------------------------
-// Routing runs in teams: one team of 4 waves per token for T = 1, two teams
-// of 2 waves for T = 2, four one-wave teams otherwise (tokens in passes).
+// ---- one-token front kernel LDS layout (dwords) --------------------------------------
+constexpr int kFrontThreads = 256, kFrontWaves = 4;
 
-__host__ __device__ constexpr FrontLds front_lds(int T, int nbh, int E, int k, bool routed) {
+__host__ __device__ constexpr FrontLds front_lds(int nbh, int E, int k, bool routed) {
   FrontLds L{};
-  L.nteams = T == 1 ? 1 : (T == 2 ? 2 : 4);
-  L.tw = 4 / L.nteams;
-  L.TT = 64 * L.tw;
-  L.ept = (E + L.TT - 1) / L.TT;
+  L.ept = (E + kFrontThreads - 1) / kFrontThreads;
   L.m = k + 1;
   L.e32 = (E + 31) & ~31;
-  L.ncp = (L.tw * L.m + 3) & ~3;  // a team's candidates: m per wave
-  const int gmax = (T * k < E ? T * k : E) + 1;
+  L.ncp = (kFrontWaves * L.m + 3) & ~3;  // the candidates: m per wave
+  const int gmax = (k < E ? k : E) + 1;
   int o = 0;
   auto take = [&](int words) {
     o = (o + 3) & ~3;  // 16-B alignment for every array
@@ -149,27 +145,26 @@ __host__ __device__ constexpr FrontLds front_lds(int T, int nbh, int E, int k, b
     o += words;
     return at;
   };
-  L.xs = take(T * nbh * kXStride);
+  L.xs = take(nbh * kXStride);
   if (routed) {
     L.tabg = take(E * 2);
     L.tabu = take(E * 2);
     L.tabd = take(E * 2);
-    L.lv = take(L.nteams * L.e32);
-    L.ev = take(4 * L.e32);  // a team's (one token) or a wave's (routing launch) exps
-    L.cand = take(L.nteams * L.ncp * 2);
-    L.top = take(L.nteams * L.m * 2);
-    L.red = take(L.nteams * 4);
-    L.zs = take(L.nteams);
-    L.spec = take(T * L.m);
-    L.ridx = take(T * k);
-    L.rw = take(T * (k + 1));
-    L.re = take(T * k);
-    L.rfirst = take(T * k);
+    L.lv = take(L.e32);
+    L.ev = take(L.e32);
+    L.cand = take(L.ncp * 2);
+    L.top = take(L.m * 2);
+    L.red = take(4);
+    L.zs = take(1);
+    L.ridx = take(k);
+    L.rw = take(k + 1);
+    L.re = take(k);
+    L.rfirst = take(k);
     L.poff = take(gmax + 1);
     L.pexp = take(gmax);
-    L.ptok = take(T * k + T);
-    L.pslot = take(T * k + T);
-    L.ctrl = take(8 + T * k);
+    L.ptok = take(k + 1);
+    L.pslot = take(k + 1);
+    L.ctrl = take(4);
     L.kw = take(4 * 64 + 4 * 128);  // team_select, one key per thread: value words, then keys
   }
   L.total = o;
@@ -201,9 +196,7 @@ __device__ __forceinline__ int rank_n(const uint64_t* c, int n, uint64_t key) {
   return r;
 }
 
-constexpr int kWaves4 = 4;  // waves of a front workgroup
-
-// Top-m selection of a team (tw waves) over the keys kr[] its threads hold
+// Top-m selection of the workgroup (a team of four waves) over the keys kr[] its threads hold
 // (0 = no key; keys are otherwise distinct).  Stage 1, per wave: the wave's
 // m largest keys go to cand[wave * m ...) (zero-padded).  With one key per
 // thread each key takes its rank among the wave's 64 keys, read back from
@@ -211,8 +204,8 @@ constexpr int kWaves4 = 4;  // waves of a front workgroup
 // bitwise radix search over ballot counts finds the wave's m-th largest key
 // - first on the value word, then, only when several keys share the
 // boundary value, on the index word.  Stage 2: each candidate's rank among
-// the team's tw*m candidates places it in top[rank] (0 = missing); when
-// they fit one wave every wave of the team does this and writes the same
+// the 4 m candidates places it in top[rank] (0 = missing); when
+// they fit one wave every wave does this and writes the same
 // top[], so it is readable by each wave on return after one barrier,
 // otherwise the candidates are shared out and a second barrier follows.
 // Every thread of the workgroup takes part.
@@ -264,7 +257,7 @@ __device__ __forceinline__ void team_select(const FrontLds& L, const uint64_t* k
     typedef __attribute__((address_space(3))) volatile uint64_t lds_vu64;
     const bool lost = place && ((lds_vu64*)(wc))[r] != kr[0];
     if (__ballot(lost)) {
-      uint64_t* kw = reinterpret_cast<uint64_t*>(kwbase + 64 * kWaves4) + 64 * (threadIdx.x >> 6);
+      uint64_t* kw = reinterpret_cast<uint64_t*>(kwbase + 64 * kFrontWaves) + 64 * (threadIdx.x >> 6);
       kw[lane] = kr[0];
       const u32x4* p2 = reinterpret_cast<const u32x4*>(kw);
       r = 0;
@@ -317,7 +310,7 @@ __device__ __forceinline__ void team_select(const FrontLds& L, const uint64_t* k
     }
   }
   if (lane >= base && lane < m) wc[lane] = 0;
-  const int nc = L.tw * m;
+  const int nc = kFrontWaves * m;
   if (tt >= nc && tt < L.ncp) cand[tt] = 0;  // rank_n reads whole 16-B pairs
   if (tt < m) top[tt] = 0;
   if (wait_before_rank) wait_vm();  // the caller's copies are visible after the barrier
@@ -344,12 +337,11 @@ __device__ __forceinline__ void team_select(const FrontLds& L, const uint64_t* k
   }
 }
 
-// Expert-major plan from ridx[T*k] (ids outside [0, E) skipped): group 0 =
-// shared expert when present, then distinct routed experts ascending;
-// entries in (expert, token, slot) order.  ctrl[0] = valid routes,
-// ctrl[1] = distinct experts.  Runs on wave 0 when T*k <= 64 (cross-lane
-// reads), else on the whole workgroup; ends with a workgroup barrier.
-__device__ __forceinline__ void build_plan(uint32_t* dyn, const FrontLds& L, int T, int k, int E, int has_shared,
+// Expert-major plan of one token from ridx[k] (ids outside [0, E) skipped):
+// group 0 = shared expert when present, then distinct routed experts
+// ascending; entries in (expert, slot) order.  ctrl[0] = valid routes,
+// ctrl[1] = distinct experts.  Runs on wave 0; ends with a workgroup barrier.
+__device__ __forceinline__ void build_plan(uint32_t* dyn, const FrontLds& L, int k, int E, int has_shared,
                            int tid) {
   const int* ridx = reinterpret_cast<const int*>(dyn + L.ridx);
   int* re = reinterpret_cast<int*>(dyn + L.re);
@@ -359,111 +351,63 @@ __device__ __forceinline__ void build_plan(uint32_t* dyn, const FrontLds& L, int
   int* ptok = reinterpret_cast<int*>(dyn + L.ptok);
   int* pslot = reinterpret_cast<int*>(dyn + L.pslot);
   int* ctrl = reinterpret_cast<int*>(dyn + L.ctrl);
-  const int R = T * k;
-  const int gbase = has_shared, ebase = has_shared ? T : 0;
-  if (R <= 64) {
-    if (tid < 64) {
-      // One wave sorts the routes by key = (expert, route index): each
-      // lane's rank is the count of smaller keys, read back from LDS with
-      // broadcast 16-B reads (the wave's own writes, visible to its later
-      // reads without a barrier).  Keys are below 2^17, so the comparison
-      // is the sign bit of an integer difference (no lane masks).  An
-      // invalid id sorts last and is left out.  Then the sorted keys come
-      // back in lane order: lane r holds the r-th entry, its expert starts
-      // a group when the previous entry's differs, and its group is the
-      // count of group starts below it (a ballot).
-      const int lane = tid;
-      int e = lane < R ? ridx[lane] : -1;
-      if (e < 0 || e >= E) e = -1;
-      if (lane < R) re[lane] = e;
-      const int key = lane < R ? (e >= 0 ? e : 1024) * 64 + lane : 0x7FFFFFFF;
-      int* keys = rfirst;  // the sort's scratch: R keys, then the sorted ones
-      if (lane < R) keys[lane] = key;
-      int rank = 0;
-      for (int j0 = 0; j0 < R; j0 += 4) {
-        const int4 v = *reinterpret_cast<const int4*>(keys + j0);
-        const int kv4[4] = {v.x, v.y, v.z, v.w};
+  const int gbase = has_shared, ebase = has_shared;
+  if (tid < 64) {
+    // The wave sorts the routes by key = (expert, slot): each lane's rank is
+    // the count of smaller keys, read back from LDS with broadcast 16-B reads
+    // (the wave's own writes, visible to its later reads without a barrier).
+    // Keys are below 2^17, so the comparison is the sign bit of an integer
+    // difference (no lane masks).  An invalid id sorts last and is left out.
+    // Then the sorted keys come back in lane order: lane r holds the r-th
+    // entry, its expert starts a group when the previous entry's differs, and
+    // its group is the count of group starts below it (a ballot).
+    const int lane = tid;
+    int e = lane < k ? ridx[lane] : -1;
+    if (e < 0 || e >= E) e = -1;
+    if (lane < k) re[lane] = e;
+    const int key = lane < k ? (e >= 0 ? e : 1024) * 64 + lane : 0x7FFFFFFF;
+    int* keys = rfirst;  // the sort's scratch: k keys, then the sorted ones
+    if (lane < k) keys[lane] = key;
+    int rank = 0;
+    for (int j0 = 0; j0 < k; j0 += 4) {
+      const int4 v = *reinterpret_cast<const int4*>(keys + j0);
+      const int kv4[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-          if (j0 + u < R)
-            rank += static_cast<int>(__builtin_amdgcn_ubfe(static_cast<unsigned>(kv4[u] - key), 31, 1));
-      }
-      int* sorted = ptok;  // placed here, then overwritten below with the entries' tokens
-      const int nv = __popcll(__ballot(e >= 0));
-      if (lane < R) sorted[rank] = key;
-      const int sk = lane < nv ? sorted[lane] : 0;
-      const int sp = lane > 0 && lane < nv ? sorted[lane - 1] : -64;
-      const int se = sk >> 6, si = sk & 63;
-      const bool first = lane < nv && (lane == 0 || (sp >> 6) != se);
-      const uint64_t fm = __ballot(first);
-      const int grp = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(fm >> 32),
-                                                __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(fm), 0));
-      const int nf = __popcll(fm);
-      wait_lds();  // the sorted keys are read before the entries overwrite them
-      if (lane < nv) {
-        ptok[ebase + lane] = si / k;
-        pslot[ebase + lane] = si % k;
-        if (first) {
-          poff[gbase + grp] = ebase + lane;
-          pexp[gbase + grp] = se;
-        }
-      }
-      if (has_shared && lane < T) {
-        ptok[lane] = lane;
-        pslot[lane] = k;
-      }
-      if (lane == 0) {
-        poff[0] = 0;
-        poff[gbase + nf] = ebase + nv;
-        if (has_shared) pexp[0] = -1;
-        ctrl[0] = nv;
-        ctrl[1] = nf;
+      for (int u = 0; u < 4; ++u)
+        if (j0 + u < k)
+          rank += static_cast<int>(__builtin_amdgcn_ubfe(static_cast<unsigned>(kv4[u] - key), 31, 1));
+    }
+    int* sorted = ptok;  // placed here, then overwritten below with the entries' tokens
+    const int nv = __popcll(__ballot(e >= 0));
+    if (lane < k) sorted[rank] = key;
+    const int sk = lane < nv ? sorted[lane] : 0;
+    const int sp = lane > 0 && lane < nv ? sorted[lane - 1] : -64;
+    const int se = sk >> 6, si = sk & 63;
+    const bool first = lane < nv && (lane == 0 || (sp >> 6) != se);
+    const uint64_t fm = __ballot(first);
+    const int grp = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(fm >> 32),
+                                              __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(fm), 0));
+    const int nf = __popcll(fm);
+    wait_lds();  // the sorted keys are read before the entries overwrite them
+    if (lane < nv) {
+      ptok[ebase + lane] = 0;
+      pslot[ebase + lane] = si;
+      if (first) {
+        poff[gbase + grp] = ebase + lane;
+        pexp[gbase + grp] = se;
       }
     }
-    bar();
-    return;
-  }
-  if (tid == 0) ctrl[0] = ctrl[1] = 0;
-  for (int i = tid; i < R; i += 256) {
-    const int e = ridx[i];
-    re[i] = (e >= 0 && e < E) ? e : -1;
-  }
-  bar();
-  for (int i = tid; i < R; i += 256) {
-    const int e = re[i];
-    int first = e >= 0;
-    for (int j = 0; j < i && first; ++j) first = re[j] != e;
-    rfirst[i] = first;
-    if (e >= 0) atomicAdd(&ctrl[0], 1);
-    if (first) atomicAdd(&ctrl[1], 1);
-  }
-  bar();
-  for (int i = tid; i < R; i += 256) {
-    const int e = re[i];
-    if (e < 0) continue;
-    int rank = 0, grp = 0;
-    for (int j = 0; j < R; ++j) {
-      const int ej = re[j];
-      if (ej < 0) continue;
-      rank += ej < e || (ej == e && j < i);
-      grp += rfirst[j] && ej < e;
+    if (lane == 0) {
+      if (has_shared) {
+        ptok[0] = 0;
+        pslot[0] = k;
+        pexp[0] = -1;
+      }
+      poff[0] = 0;
+      poff[gbase + nf] = ebase + nv;
+      ctrl[0] = nv;
+      ctrl[1] = nf;
     }
-    ptok[ebase + rank] = i / k;
-    pslot[ebase + rank] = i % k;
-    if (rfirst[i]) {
-      poff[gbase + grp] = ebase + rank;
-      pexp[gbase + grp] = e;
-    }
-  }
-  if (has_shared && tid < T) {
-    ptok[tid] = tid;
-    pslot[tid] = k;
-  }
-  bar();
-  if (tid == 0) {
-    poff[0] = 0;
-    poff[gbase + ctrl[1]] = ebase + ctrl[0];
-    if (has_shared) pexp[0] = -1;
   }
   bar();
 }
@@ -704,58 +648,36 @@ __device__ __forceinline__ void quantize_x(const LayerArgs& a, int n_blocks, uin
   }
 }
 
-// Logit-order top-(k+1) of every token: spec[t*m + r] = r-th expert (or -1).
-// Logits of the first routing pass into lr[] (what spec_select's pass 0
-// reads): thread tt of team `team` holds experts tt + TT*j of token `team`,
-// 0 outside.  Same team geometry as front_lds.
+// The token's logits into lr[]: thread tid holds experts tid + 256 j, 0 outside.
 template <int EPT>
-__device__ __forceinline__ void logits_preload(const LayerArgs& a, int T, int tid, float* lr) {
+__device__ __forceinline__ void logits_preload(const LayerArgs& a, int tid, float* lr) {
   const int E = a.n_expert;
-  const int nteams = T == 1 ? 1 : (T == 2 ? 2 : 4);
-  const int TT = 64 * (4 / nteams);
-  const int ept = (E + TT - 1) / TT;
-  const int team = tid / TT, tt = tid - team * TT;
-  const bool ok = team < T;
-  const float* lg = a.logits + static_cast<long long>(team) * E;
+  const int ept = (E + kFrontThreads - 1) / kFrontThreads;
 #pragma unroll
   for (int j = 0; j < EPT; ++j) {
-    const int i = tt + TT * j;
-    lr[j] = (j < ept && i < E && ok) ? lg[i] : 0.f;
+    const int i = tid + kFrontThreads * j;
+    lr[j] = (j < ept && i < E) ? a.logits[i] : 0.f;
   }
 }
 
-// Logit-order top-(k+1) of every token: teams of tw waves, one token per
-// team per pass; each thread keeps its logits in lr[] (pass 0's from
-// logits_preload, then the last pass's token).  Workgroup-wide; the last
-// pass's top[] is readable on return, spec[] only after the caller's next
-// barrier.  wait_copies: the calling wave waits for its outstanding copies
-// before the selection's barrier (so they are visible on return).
+// Logit-order top-(k+1): top[], readable on return, and the logits in lv[].
+// wait_copies: the calling wave waits for its outstanding copies before the
+// selection's barrier (so they are visible on return).
 template <int EPT>
-__device__ __forceinline__ void spec_select(const LayerArgs& a, int T, uint32_t* dyn, const FrontLds& L,
-                            float* lr, int tid, bool wait_copies = false) {
-  const int E = a.n_expert, m = L.m;
-  const int wave = tid >> 6, team = wave / L.tw, tt = tid - team * L.TT;
-  float* lv = reinterpret_cast<float*>(dyn + L.lv) + team * L.e32;
-  uint64_t* cand = reinterpret_cast<uint64_t*>(dyn + L.cand) + team * L.ncp;
-  uint64_t* top = reinterpret_cast<uint64_t*>(dyn + L.top) + team * m;
-  int* spec = reinterpret_cast<int*>(dyn + L.spec);
-  for (int t0 = 0; t0 < T; t0 += L.nteams) {
-    const int t = t0 + team;
-    const bool ok = t < T;
-    const float* lg = a.logits + static_cast<long long>(t) * E;
-    uint64_t kr[EPT];
+__device__ __forceinline__ void spec_select(const LayerArgs& a, uint32_t* dyn, const FrontLds& L,
+                            const float* lr, int tid, bool wait_copies = false) {
+  const int E = a.n_expert;
+  float* lv = reinterpret_cast<float*>(dyn + L.lv);
+  uint64_t* cand = reinterpret_cast<uint64_t*>(dyn + L.cand);
+  uint64_t* top = reinterpret_cast<uint64_t*>(dyn + L.top);
+  uint64_t kr[EPT];
 #pragma unroll
-    for (int j = 0; j < EPT; ++j) {
-      const int i = tt + L.TT * j;
-      const bool in = j < L.ept && i < E && ok;
-      if (t0 > 0) lr[j] = in ? lg[i] : 0.f;  // pass 0: logits_preload
-      kr[j] = in ? sel_key(lr[j], i) : 0;
-      if (j < L.ept && i < L.e32) lv[i] = lr[j];
-    }
-    team_select<EPT>(L, kr, cand, top, dyn + L.kw, tt, wait_copies && t0 == 0);
-    if (ok && tt < m) spec[t * m + tt] = top[tt] ? sel_idx(top[tt]) : -1;
-    if (t0 + L.nteams < T) bar();  // the next pass reuses cand/top
+  for (int j = 0; j < EPT; ++j) {
+    const int i = tid + kFrontThreads * j;
+    kr[j] = j < L.ept && i < E ? sel_key(lr[j], i) : 0;
+    if (j < L.ept && i < L.e32) lv[i] = lr[j];
   }
+  team_select<EPT>(L, kr, cand, top, dyn + L.kw, tid, wait_copies);
 }
 
 // Plan for T == 1 straight from k distinct, valid ids id(0..k-1): group
@@ -806,15 +728,15 @@ __device__ __forceinline__ bool ids_distinct_valid(const int* ridx, int n, int E
   return ok;
 }
 
-// The plan of ridx[0..T*k): the one-token form when the ids are distinct
-// and valid, else the general build.  Ends with a barrier.
-__device__ __forceinline__ void make_plan(uint32_t* dyn, const FrontLds& L, int T, int k, int E,
+// The plan of ridx[0..k): the direct form when the ids are distinct and
+// valid, else the general build.  Ends with a barrier.
+__device__ __forceinline__ void make_plan(uint32_t* dyn, const FrontLds& L, int k, int E,
                                           int has_shared, int tid) {
   const int* ridx = reinterpret_cast<const int*>(dyn + L.ridx);
-  if (T == 1 && ids_distinct_valid(ridx, k, E))
+  if (ids_distinct_valid(ridx, k, E))
     plan_t1(dyn, L, k, has_shared, tid, [&](int j) { return ridx[j]; });
   else
-    build_plan(dyn, L, T, k, E, has_shared, tid);
+    build_plan(dyn, L, k, E, has_shared, tid);
 }
 
 // Whether the exact routing of one token (route_wave) is sure to select the
@@ -850,7 +772,10 @@ __device__ __forceinline__ bool route_is_logit_order(const LayerArgs& a, const u
 }
 
 // Exact routing of ONE token by one wave, no workgroup barrier (moe.cu:25-85):
-// same arithmetic and checks as exact_route below.  Logits come from lv[]
+// max, exp, the normalizer summed serially in index order, p = e / z, and the
+// check that p is strictly decreasing along the logit order (or equal logits);
+// a collision selects on the probabilities, a degenerate row (NaN, empty
+// normalizer) takes kk % E with weight -1.  Logits come from lv[]
 // (LDS, filled by spec_select), lane l holds experts l + 64j.  Writes ridx,
 // rw and ctrl[3] (1 when an id differs from the logit order).
 template <int EPL>
@@ -956,12 +881,12 @@ __device__ __forceinline__ void route_direct_t1(const LayerArgs& a, uint32_t* dy
   float mx = -1e30f;
 #pragma unroll
   for (int j = 0; j < EPT; ++j)
-    if (j < L.ept && tid + L.TT * j < E) mx = fmaxf(mx, lr[j]);
-  mx = team_max(mx, red, wave, L.tw, lane);
+    if (j < L.ept && tid + kFrontThreads * j < E) mx = fmaxf(mx, lr[j]);
+  mx = team_max(mx, red, wave, kFrontWaves, lane);
   float e[EPT];
 #pragma unroll
   for (int j = 0; j < EPT; ++j) {
-    const int i = tid + L.TT * j;
+    const int i = tid + kFrontThreads * j;
     e[j] = (j < L.ept && i < E) ? expf_sg(lr[j] - mx) : 0.f;
     if (j < L.ept && i < L.e32) ev[i] = e[j];
   }
@@ -974,7 +899,7 @@ __device__ __forceinline__ void route_direct_t1(const LayerArgs& a, uint32_t* dy
     uint64_t kr[EPT];
 #pragma unroll
     for (int j = 0; j < EPT; ++j) {
-      const int i = tid + L.TT * j;
+      const int i = tid + kFrontThreads * j;
       kr[j] = (j < L.ept && i < E) ? sel_key(e[j] / z, i) : 0ull;
     }
     team_select<EPT>(L, kr, cand, top, dyn + L.kw, tid);
@@ -1027,132 +952,13 @@ __device__ __forceinline__ void route_direct_t1(const LayerArgs& a, uint32_t* dy
   bar();
 }
 
-// Exact routing of every token (moe.cu:25-85): max, exp, the normalizer
-// summed serially in index order, p = e / z.  p is a monotone function of
-// the logit, so the logit order (spec[]) is the probability order unless two
-// neighbours collide on one float; the check is p strictly decreasing
-// across the k+1 leading candidates (or equal logits).  A collision selects
-// on the probabilities themselves; a degenerate row (NaN, empty normalizer)
-// takes kk % E with weight -1.  Writes ridx (replacing the logit-order ids)
-// and rw; ctrl[3] = 1 when any id changed.  Workgroup-wide, barriers only
-// (no wait on the weight stream in flight).
-template <int EPT>
-__device__ __forceinline__ void exact_route(const LayerArgs& a, uint32_t* dyn, const FrontLds& L, float* lr,
-                            int tid) {
-  const int T = a.T, E = a.n_expert, k = a.k, stride = k + 1, m = L.m;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int tw = L.tw, team = wave / tw, wit = wave - team * tw;
-  const int tt = tid - team * L.TT;
-  float* lv = reinterpret_cast<float*>(dyn + L.lv) + team * L.e32;
-  float* ev = reinterpret_cast<float*>(dyn + L.ev) + team * L.e32;
-  uint64_t* cand = reinterpret_cast<uint64_t*>(dyn + L.cand) + team * L.ncp;
-  uint64_t* top = reinterpret_cast<uint64_t*>(dyn + L.top) + team * m;
-  float* red = reinterpret_cast<float*>(dyn + L.red) + team * 4;
-  float* zs = reinterpret_cast<float*>(dyn + L.zs);
-  int* spec = reinterpret_cast<int*>(dyn + L.spec);
-  int* ridx = reinterpret_cast<int*>(dyn + L.ridx);
-  float* rw = reinterpret_cast<float*>(dyn + L.rw);
-  int* ctrl = reinterpret_cast<int*>(dyn + L.ctrl);
-  if (tid == 0) ctrl[3] = 0;
-  for (int t0 = 0; t0 < T; t0 += L.nteams) {
-    const int t = t0 + team;
-    const bool ok = t < T;
-    if (T > L.nteams) {  // several passes: (re)load this token's logits
-      const float* lg = a.logits + static_cast<long long>(t) * E;
-#pragma unroll
-      for (int j = 0; j < EPT; ++j) {
-        const int i = tt + L.TT * j;
-        lr[j] = (j < L.ept && i < E && ok) ? lg[i] : 0.f;
-        if (j < L.ept && i < L.e32) lv[i] = lr[j];
-      }
-    }
-    if (tid == 0) ctrl[2] = 0;
-    float mx = -1e30f;
-#pragma unroll
-    for (int j = 0; j < EPT; ++j)
-      if (j < L.ept && tt + L.TT * j < E && ok) mx = fmaxf(mx, lr[j]);
-    mx = team_max(mx, red, wit, tw, lane);
-#pragma unroll
-    for (int j = 0; j < EPT; ++j) {
-      const int i = tt + L.TT * j;
-      if (j < L.ept && i < L.e32) ev[i] = (ok && i < E) ? expf_sg(lr[j] - mx) : 0.f;
-    }
-    bar();
-    if (tt == 0) zs[team] = serial_sum(ev, L.e32);
-    bar();
-    const float z = zs[team];
-    const bool degen = !(z == z) || z == 0.f;
-    bool fast = false;
-    float pk = -1.f;
-    int ik = -1;
-    if (wit == 0) {
-      ik = (ok && lane < m) ? spec[t * m + lane] : -1;
-      pk = (ik >= 0 && !degen) ? ev[ik] / z : -1.f;
-      const float lk = ik >= 0 ? lv[ik] : 0.f;
-      const float pn = __shfl(pk, lane + 1, 64);
-      const float ln = __shfl(lk, lane + 1, 64);
-      const int in = __shfl(ik, lane + 1, 64);
-      bool cond = true;
-      if (lane + 1 < k) cond = ik >= 0 && in >= 0 && (pk > pn || lk == ln);
-      else if (lane + 1 == k && E > k) cond = ik >= 0 && in >= 0 && pk > pn;
-      fast = ok && !degen && __ballot(!cond) == 0;
-      if (lane == 0) {
-        ctrl[4 + team] = ok && !degen && !fast;
-        if (ok && !degen && !fast) atomicOr(&ctrl[2], 1);
-      }
-    }
-    bar();
-    if (ctrl[2] != 0) {  // selection on the probabilities for the colliding rows
-      const bool slow_team = ctrl[4 + team] != 0;
-      uint64_t kr[EPT];
-#pragma unroll
-      for (int j = 0; j < EPT; ++j) {
-        const int i = tt + L.TT * j;
-        kr[j] = (j < L.ept && i < E && slow_team) ? sel_key(ev[i] / z, i) : 0;
-      }
-      team_select<EPT>(L, kr, cand, top, dyn + L.kw, tt);
-    }
-    if (wit == 0 && ok) {
-      int fi;
-      float pv;
-      if (degen) {
-        fi = lane % E;
-        pv = -1.f;
-      } else if (fast) {
-        fi = ik;
-        pv = pk;
-      } else {
-        fi = lane < m && top[lane] ? sel_idx(top[lane]) : 0;
-        pv = ev[fi] / z;
-      }
-      float wsum = 0.f;
-      for (int kk = 0; kk < k; ++kk) wsum += readlane_f(pv, kk);
-      const float wv = wsum > 0.f ? pv / wsum : pv;
-      if (lane < k) {
-        if (fi != ridx[t * k + lane]) atomicOr(&ctrl[3], 1);
-        ridx[t * k + lane] = fi;
-        rw[t * stride + lane] = wv;
-      }
-      if (lane == 0) rw[t * stride + k] = a.shared_w;
-    }
-    bar();
-  }
-}
-
-// Compute workgroups (blockIdx.y < gmax): one (group, chunk of 16 rows).
-// The shared expert's group streams at once; a routed group streams the
-// expert the logit order gives it, then checks that against the exact
-// routing (streaming the exact expert instead when they differ) and writes
-// h for the (token, slot) entries of its group in the exact plan.  The
-// publisher workgroup (blockIdx.y == gmax, x == 0) runs the same routing
-// and writes idx, weight and the plan.
-// NBH: hidden / 256 when compiled for it (0 = read from a).
 // The shared expert's scalar gate of every token (session.cpp:2904-2909),
 // sgate[t] = sigmoid(sh_gate_w . x[t]) in the reference's fp32 lane order:
-// one token per 32-lane half-wave of the workgroup; read by the back kernel.
-__device__ __forceinline__ void shared_gate_tokens(const LayerArgs& a, int tid) {
+// one token per 32-lane half-wave of the workgroup (n_halves of them); read
+// by the back kernel.
+__device__ __forceinline__ void shared_gate_tokens(const LayerArgs& a, int tid, int n_halves) {
   const int l = tid & 31, half = tid >> 5;
-  for (int t0 = 0; t0 < a.T; t0 += 8) {
+  for (int t0 = 0; t0 < a.T; t0 += n_halves) {
     const int t = min(t0 + half, a.T - 1);
     const long long o = static_cast<long long>(t) * a.hidden;
     const float gl =
@@ -1162,16 +968,26 @@ __device__ __forceinline__ void shared_gate_tokens(const LayerArgs& a, int tid) 
   }
 }
 
-// kOne: the one-token decode instance (T = 1 at compile time, so the
-// several-token paths are not compiled into it)
-template <int EPT, int NBH, bool kOne>
+// One token.  Compute workgroups (group g < gmax): one (group, chunk of 16
+// rows).  The shared expert's group streams at once; a routed group streams
+// the expert the logit order gives it, then checks that against the exact
+// routing (streaming the exact expert instead when they differ) and writes
+// h for the entry of its group in the exact plan.  The publisher workgroup
+// (g == gmax, bx == 0) runs the same routing and writes idx, weight and the
+// plan; the next one of its row (bx == 1), otherwise idle, computes the shared
+// expert's gate.
+// NBH: hidden / 256 when compiled for it (0 = read from a).
+template <int EPT, int NBH>
 __device__ __forceinline__ void front_body(const LayerArgs& a, int bx, int g, uint32_t (*wbuf)[64 * 36],
                            uint32_t* dyn) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int T = kOne ? 1 : a.T, k = a.k, E = a.n_expert, stride = k + 1;
+  const int k = a.k, E = a.n_expert, stride = k + 1;
   const int nbh = NBH ? NBH : a.hidden / kQK, lpr = NBH ? pow2_ceil(NBH) : pow2_ceil(nbh);
   const bool publisher = g == a.gmax;
-  if (publisher && bx != 0) return;  // one publisher per launch
+  if (publisher && bx != 0) {  // one publisher per launch
+    if (bx == 1 && a.sh_gate_w) shared_gate_tokens(a, tid, kFrontThreads / 32);
+    return;
+  }
   const bool shared_grp = a.has_shared && g == 0;
   const bool tabd_regs = publisher && E <= 256;
   // expert pointer tables into LDS (gate and up; down for the publisher),
@@ -1195,9 +1011,9 @@ __device__ __forceinline__ void front_body(const LayerArgs& a, int bx, int g, ui
     else
       copy_table(a.tab_down, a.front_routed.tabd);
   }
-  // the first routing pass's logits are the head of the routing chain
+  // the logits are the head of the routing chain
   float lr[EPT];
-  if (a.logits && !shared_grp) logits_preload<EPT>(a, T, tid, lr);
+  if (a.logits && !shared_grp) logits_preload<EPT>(a, tid, lr);
   const FrontLds& L = shared_grp ? a.front_shared : a.front_routed;
   const int rpw = 32 / lpr;
   const int row0 = bx * 4 * rpw + wave * rpw;
@@ -1208,10 +1024,10 @@ __device__ __forceinline__ void front_body(const LayerArgs& a, int bx, int g, ui
   const int gbase = a.has_shared;
   uint32_t* buf = wbuf[wave];
   uint32_t* xs = dyn + L.xs;
-  const int nxb = T * nbh;
-  // one token with router logits: wave 3 does the exact routing on its own
-  // while waves 0-2 issue the weight stream and quantize x
-  const bool t1w = T == 1 && a.logits != nullptr && !shared_grp;
+  const int nxb = nbh;
+  // with router logits wave 3 does the exact routing on its own while waves
+  // 0-2 issue the weight stream and quantize x
+  const bool t1w = a.logits != nullptr && !shared_grp;
   const int nqw = t1w ? 3 : 4;
   float xpre[1][16];
   if (!publisher) x_preload(a, nxb, wave, nqw, lane, xpre);
@@ -1220,11 +1036,12 @@ __device__ __forceinline__ void front_body(const LayerArgs& a, int bx, int g, ui
     if (nrw > 0) dma_gateup(a.sh_gate, a.sh_up, row0, nrw, nbh, buf, lane);
     quantize_x(a, nxb, xs, wave, nqw, lane, xpre);
     bar();
-    // entries: tokens 0..T-1 in slot k, no plan needed
+    // its entry is the token in slot k: no plan needed
     gateup_wave(true, row0, nrw, nbh, lpr, buf, xs,
-                [&](int j, int& t, int& sl) { t = j; sl = k; }, T, stride, a.n_ff, a.h, lane,
+                [&](int, int& t, int& sl) { t = 0; sl = k; }, 1, stride, a.n_ff, a.h, lane,
                 a.out16 != nullptr);
-    if (a.sh_gate_w && bx == 0) shared_gate_tokens(a, tid);
+    // (a grid of one row chunk has no idle publisher-row workgroup)
+    if (a.sh_gate_w && gridDim.x == 1) shared_gate_tokens(a, tid, kFrontThreads / 32);
     return;
   }
 
@@ -1232,7 +1049,6 @@ __device__ __forceinline__ void front_body(const LayerArgs& a, int bx, int g, ui
   const unsigned long long* tabu = reinterpret_cast<const unsigned long long*>(dyn + L.tabu);
   const unsigned long long* tabd = reinterpret_cast<const unsigned long long*>(dyn + L.tabd);
   int* ridx = reinterpret_cast<int*>(dyn + L.ridx);
-  int* spec = reinterpret_cast<int*>(dyn + L.spec);
   float* rw = reinterpret_cast<float*>(dyn + L.rw);
   int* ctrl = reinterpret_cast<int*>(dyn + L.ctrl);
   const int* pexp = reinterpret_cast<const int*>(dyn + L.pexp);
@@ -1267,28 +1083,7 @@ __device__ __forceinline__ void front_body(const LayerArgs& a, int bx, int g, ui
   int e_mine = -1, slot_mine = -1;
   bool present_mine = false;
   int n_groups;
-  if (a.logits && publisher && T > 1) {
-    // the routing launch of several tokens: one wave per token, each the
-    // standalone router's exact routing (router_wave), then the plan
-    // experts per lane: E <= 64 PL (the launch picks EPT with E <= 64 EPT
-    // for three or more tokens, E <= 128 EPT for two)
-    constexpr int kPl1 = EPT < 16 ? EPT : 16, kPl2 = 2 * EPT < 16 ? 2 * EPT : 16;
-    float* evw = reinterpret_cast<float*>(dyn + L.ev) + wave * L.e32;
-    // x of the window for waves 1-3 to quantize while wave 0 builds the plan
-    float xw[3][16];
-    if (wave > 0) x_preload(a, nxb, wave - 1, 3, lane, xw);
-    for (int t = wave; t < T; t += 4) {
-      const float* lg = a.logits + static_cast<long long>(t) * E;
-      if (T == 2)
-        router_wave<kPl2>(lg, E, k, a.shared_w, ridx + t * k, rw + t * stride, evw, lane);
-      else
-        router_wave<kPl1>(lg, E, k, a.shared_w, ridx + t * k, rw + t * stride, evw, lane);
-    }
-    bar();
-    if (wave > 0) quantize_x(a, nxb, a.xq, wave - 1, 3, lane, xw);
-    build_plan(dyn, L, T, k, E, a.has_shared, tid);
-    n_groups = gbase + ctrl[1];
-  } else if (a.logits && publisher && T == 1) {
+  if (a.logits && publisher) {
     // the publisher routes exactly from the logits with every wave; it has
     // no stream to start and needs the weights, not the logit order
     route_direct_t1<EPT>(a, dyn, L, lr, tid);  // and the plan
@@ -1296,101 +1091,73 @@ __device__ __forceinline__ void front_body(const LayerArgs& a, int bx, int g, ui
   } else if (a.logits) {
     // waves 0-1 wait for the pointer tables inside the selection, so they
     // are readable when it returns
-    spec_select<EPT>(a, T, dyn, L, lr, tid, wave < 2);
-    bool streamed = false, routed = false;
-    if (T == 1) {
-      // top[] of the single token is readable now: with k valid ids the
-      // plan is made here, in the same phase as spec[] and ridx[]
-      const uint64_t* top = reinterpret_cast<const uint64_t*>(dyn + L.top);
-      const uint64_t tk = lane < k ? top[lane] : 1ull;  // lane j: key of slot j
-      const bool valid = __ballot(tk == 0ull) == 0ull;
-      if (valid) {
-        if (!publisher) {
-          // speculative: the logit-order expert of this group, i.e. the one
-          // of id rank g - gbase among top[] (what plan_t1 assigns), and its
-          // slot, read straight from top[] so the stream starts before the
-          // plan round.  Waves 0-2 issue it (each also a third of wave 3's
-          // rows) so wave 3 routes unblocked.
-          const int want = g - gbase;
-          const int idl = lane < k ? sel_idx(tk) : 0x7FFFFFFF;
-          // its rank among the k ids, which every lane reads from top[]
-          // (broadcast reads; ids < 2^16, so a comparison is the sign bit
-          // of a difference)
-          int r = 0;
-          const uint32_t* tw = reinterpret_cast<const uint32_t*>(top);
-          for (int i = 0; i < k; ++i)
-            r += static_cast<int>(__builtin_amdgcn_ubfe(
-                static_cast<unsigned>(sel_idx(tw[2 * i]) - idl), 31, 1));
-          const uint64_t hit = __ballot(lane < k && r == want);
-          slot_mine = hit ? __builtin_ctzll(hit) : -1;
-          e_mine = hit ? __builtin_amdgcn_readlane(idl, slot_mine) : -1;
-          if (wave < 3) present_mine = stream_rows(e_mine, wave);
-          if (wave < 3) stream_rows(e_mine, 3, wave, 3);
-          if (wave == 3 && e_mine >= 0) present_mine = tabg[e_mine] != 0ull && tabu[e_mine] != 0ull;
-          streamed = true;
+    spec_select<EPT>(a, dyn, L, lr, tid, wave < 2);
+    bool streamed = false;
+    // with k valid ids the plan is made here, in the same phase as ridx[]
+    const uint64_t* top = reinterpret_cast<const uint64_t*>(dyn + L.top);
+    const uint64_t tk = lane < k ? top[lane] : 1ull;  // lane j: key of slot j
+    const bool valid = __ballot(tk == 0ull) == 0ull;
+    if (valid) {
+      // speculative: the logit-order expert of this group, i.e. the one
+      // of id rank g - gbase among top[] (what plan_t1 assigns), and its
+      // slot, read straight from top[] so the stream starts before the
+      // plan round.  Waves 0-2 issue it (each also a third of wave 3's
+      // rows) so wave 3 routes unblocked.
+      const int want = g - gbase;
+      const int idl = lane < k ? sel_idx(tk) : 0x7FFFFFFF;
+      // its rank among the k ids, which every lane reads from top[]
+      // (broadcast reads; ids < 2^16, so a comparison is the sign bit
+      // of a difference)
+      int r = 0;
+      const uint32_t* tw = reinterpret_cast<const uint32_t*>(top);
+      for (int i = 0; i < k; ++i)
+        r += static_cast<int>(__builtin_amdgcn_ubfe(
+            static_cast<unsigned>(sel_idx(tw[2 * i]) - idl), 31, 1));
+      const uint64_t hit = __ballot(lane < k && r == want);
+      slot_mine = hit ? __builtin_ctzll(hit) : -1;
+      e_mine = hit ? __builtin_amdgcn_readlane(idl, slot_mine) : -1;
+      if (wave < 3) present_mine = stream_rows(e_mine, wave);
+      if (wave < 3) stream_rows(e_mine, 3, wave, 3);
+      if (wave == 3 && e_mine >= 0) present_mine = tabg[e_mine] != 0ull && tabu[e_mine] != 0ull;
+      streamed = true;
+      // wave 3 routes exactly now (it reads top[] and lv[], complete since
+      // the selection's last barrier) and writes ridx[] itself; the plan
+      // is published by the barrier after the x quantization below.
+      // wave 2 (the one with the fewest x blocks to quantize) writes the
+      // plan, its lanes in the roles of threads 0..63
+      // (skipped when the logit order is provably the exact one: only the
+      // publisher needs the weights)
+      if (wave == 3) {
+        if (route_is_logit_order(a, dyn, L, lane)) {
+          if (lane == 0) ctrl[3] = 0;
+        } else {
+          route_wave<4 * EPT>(a, dyn, L, lane);
         }
-        // wave 3 routes exactly now (it reads top[] and lv[], complete since
-        // the selection's last barrier) and writes ridx[] itself; the plan
-        // is published by the barrier after the x quantization below.
-        // wave 2 (the one with the fewest x blocks to quantize) writes the
-        // plan, its lanes in the roles of threads 0..63
-        // (a compute workgroup skips it when the logit order is provably
-        // the exact one: only the publisher needs the weights; the
-        // publisher routes with all four waves below)
-        if (wave == 3 && !publisher) {
-          if (route_is_logit_order(a, dyn, L, lane)) {
-            if (lane == 0) ctrl[3] = 0;
-          } else {
-            route_wave<4 * EPT>(a, dyn, L, lane);
-          }
-        }
-        if (wave == 2) {
-          plan_t1(dyn, L, k, a.has_shared, lane, [&](int j) { return sel_idx(top[j]); }, false);
-          if (publisher && lane < k) ridx[lane] = sel_idx(top[lane]);  // what exact_route compares
-        }
-        routed = true;
-      } else {
-        if (tid < k) ridx[tid] = top[tid] ? sel_idx(top[tid]) : -1;
-        bar();
-        build_plan(dyn, L, T, k, E, a.has_shared, tid);
       }
+      if (wave == 2)
+        plan_t1(dyn, L, k, a.has_shared, lane, [&](int j) { return sel_idx(top[j]); }, false);
     } else {
+      if (tid < k) ridx[tid] = top[tid] ? sel_idx(top[tid]) : -1;
       bar();
-      for (int i = tid; i < T * k; i += 256) ridx[i] = spec[(i / k) * L.m + (i % k)];
-      bar();
-      build_plan(dyn, L, T, k, E, a.has_shared, tid);
-    }
-    if (!publisher && !streamed) {
+      build_plan(dyn, L, k, E, a.has_shared, tid);
+      // speculative, as above
       e_mine = g < gbase + ctrl[1] ? pexp[g] : -1;
-      // speculative: the logit-order expert.  One token: waves 0-2 issue
-      // the stream (each also a third of wave 3's rows) so wave 3 routes
-      // unblocked.
-      if (!t1w) {
-        stream_rows(e_mine, wave);
-      } else if (wave < 3) {
+      if (wave < 3) {
         stream_rows(e_mine, wave);
         stream_rows(e_mine, 3, wave, 3);
-      }
-    }
-    if (t1w && publisher) {
-      // no weight stream to overlap: the whole workgroup routes exactly (one
-      // exp per thread instead of four per lane of one wave)
-      exact_route<EPT>(a, dyn, L, lr, tid);
-    } else if (t1w) {
-      if (wave == 3) {
-        if (!routed) route_wave<4 * EPT>(a, dyn, L, lane);
       } else {
-        quantize_x(a, nxb, xs, wave, nqw, lane, xpre);  // overlaps the weight stream
-        wait_vm();  // this wave's share of wave 3's rows
+        route_wave<4 * EPT>(a, dyn, L, lane);
       }
-      bar();
-    } else {
-      exact_route<EPT>(a, dyn, L, lr, tid);
     }
+    if (wave < 3) {
+      quantize_x(a, nxb, xs, wave, nqw, lane, xpre);  // overlaps the weight stream
+      wait_vm();  // this wave's share of wave 3's rows
+    }
+    bar();
     const bool moved = ctrl[3] != 0;  // the exact routing changed an id
-    if (moved) make_plan(dyn, L, T, k, E, a.has_shared, tid);
+    if (moved) make_plan(dyn, L, k, E, a.has_shared, tid);
     if (streamed && !moved) {
-      // one token, routing as the logits ordered it: this group's expert,
+      // routing as the logits ordered it: this group's expert,
       // presence and single entry (token 0, slot_mine) are known already
       if (e_mine < 0) {
         wait_vm();
@@ -1402,25 +1169,18 @@ __device__ __forceinline__ void front_body(const LayerArgs& a, int bx, int g, ui
       return;
     }
     n_groups = gbase + ctrl[1];
-    if (!publisher) {
-      const int e_x = g < n_groups ? pexp[g] : -1;
-      if (e_x != e_mine) {  // a collision moved this group to another expert
-        wait_vm();          // the speculative stream has landed; reuse the buffers
-        bar();
-        stream_rows(e_x, wave);
-        e_mine = e_x;
-      }
+    const int e_x = g < n_groups ? pexp[g] : -1;
+    if (e_x != e_mine) {  // a collision moved this group to another expert
+      wait_vm();          // the speculative stream has landed; reuse the buffers
+      bar();
+      stream_rows(e_x, wave);
+      e_mine = e_x;
     }
   } else {
-    if (publisher && T > 1) {  // the gate/up launch reads x quantized
-      float xw[1][16];
-      x_preload(a, nxb, wave, 4, lane, xw);
-      quantize_x(a, nxb, a.xq, wave, 4, lane, xw);
-    }
-    for (int i = tid; i < T * k; i += 256) ridx[i] = a.idx[(i / k) * stride + (i % k)];
-    for (int i = tid; i < T * stride; i += 256) rw[i] = a.weight[i];
+    for (int i = tid; i < k; i += kFrontThreads) ridx[i] = a.idx[i];
+    for (int i = tid; i < stride; i += kFrontThreads) rw[i] = a.weight[i];
     bar();
-    make_plan(dyn, L, T, k, E, a.has_shared, tid);
+    make_plan(dyn, L, k, E, a.has_shared, tid);
     n_groups = gbase + ctrl[1];
     if (!publisher) {
       if (wave < 2) wait_vm();  // pointer tables
@@ -1445,19 +1205,17 @@ __device__ __forceinline__ void front_body(const LayerArgs& a, int bx, int g, ui
     const int* re = reinterpret_cast<const int*>(dyn + L.re);
     const int nv = ctrl[0];
     if (wave == 0) {
-      for (int i = lane; i < T * stride; i += 64) {
-        const int t = i / stride, q = i - t * stride;
+      for (int i = lane; i < stride; i += 64) {
         bool bad = false;  // bounds-kill: a row with an invalid id loses all its weights
-        for (int kk = 0; kk < k; ++kk) bad |= re[t * k + kk] < 0;
+        for (int kk = 0; kk < k; ++kk) bad |= re[kk] < 0;
         a.weight[i] = bad ? 0.f : rw[i];
-        if (a.logits && q < k) a.idx[i] = ridx[t * k + q];
+        if (a.logits && i < k) a.idx[i] = ridx[i];
       }
     } else if (wave == 1) {
       for (int i = lane; i <= n_groups; i += 64) {
         a.plan.off[i] = poff[i];
         if (i < n_groups) {
           const int e = pexp[i];
-          a.plan.expert[i] = e;
           const unsigned long long gp =
               e >= 0 ? tabg[e] : reinterpret_cast<unsigned long long>(a.sh_gate);
           const unsigned long long up =
@@ -1470,7 +1228,7 @@ __device__ __forceinline__ void front_body(const LayerArgs& a, int bx, int g, ui
         }
       }
     } else if (wave == 2) {
-      for (int i = lane; i < (a.has_shared ? T : 0) + nv; i += 64) {
+      for (int i = lane; i < a.has_shared + nv; i += 64) {
         a.plan.tok[i] = ptok[i];
         a.plan.slot[i] = pslot[i];
       }
@@ -1501,6 +1259,7 @@ __device__ __forceinline__ void front_body(const LayerArgs& a, int bx, int g, ui
 // top-8): its instance sees these and the LDS layout as constants.
 constexpr int kShapeHidden = 2048, kShapeFf = 512, kShapeE = 256, kShapeK = 8;
 constexpr int kShapeWindow = 4;  // the verify window's tokens (one plus three drafts)
+constexpr int kShSplit = 4;      // tokens per group of the shared expert
 
 // The model shape with kT tokens, with or without a shared expert, as the
 // launcher derives it (kT = 0: none).
@@ -1529,33 +1288,217 @@ __device__ __forceinline__ void apply_shape(LayerArgs& a) {
     a.k = kShapeK;
     a.gmax = (kT * kShapeK < kShapeE ? kT * kShapeK : kShapeE) + 1;
     a.emax = kT * kShapeK + kT;
-    a.front_routed = front_lds(kT, kShapeHidden / kQK, kShapeE, kShapeK, true);
-    a.front_shared = front_lds(kT, kShapeHidden / kQK, kShapeE, kShapeK, false);
+    a.split = kShSplit;
+    a.hq_pre = kT > 1;
+    a.front_routed = front_lds(kShapeHidden / kQK, kShapeE, kShapeK, true);
+    a.front_shared = front_lds(kShapeHidden / kQK, kShapeE, kShapeK, false);
   }
 }
 __host__ inline bool is_shape(int T, int hidden, int n_ff, int E, int k, int kT) {
   return T == kT && hidden == kShapeHidden && n_ff == kShapeFf && E == kShapeE && k == kShapeK;
 }
 
+// ---- routing launch (several tokens) ---------------------------------------------------
+// Grid: workgroup 0 routes and makes the plan, the next ones quantize x (64
+// blocks each), the last one computes the shared expert's gate.  Sixteen waves,
+// so every token of a batch has a wave to route it (router_wave, the
+// standalone router's exact routing) and every route a thread in the plan.
+//
+// The expert-major plan: routes sorted by (expert, token, slot), each one's
+// rank the count of smaller keys; distinct experts ascending, one group each.
+// The shared expert comes first, in groups of `split` tokens: a group's
+// entries run one after the other in the gate/up and back kernels, and one
+// group of every token is their longest chain (16 tokens: 69.7 us per layer
+// with one group, 65.6 with groups of 4).
+//
+// One workgroup of four waves routed its tokens in turns, built the plan by
+// counting serially over all routes, quantized x and wrote everything: 45.6 us
+// for 13 tokens, 8.4 for the window of 4; now 11.4 and 6.1, the gate's dot
+// included.
+constexpr int kRouteThreads = 1024, kRouteWaves = 16;
+static_assert(kLMaxTokens <= kRouteWaves && kLMaxTokens * kLMaxK <= kRouteThreads,
+              "a wave per token, a thread per route");
+
+struct RouteLds {
+  int tabs, ev, ridx, rw, keys, sorted, cnt, total;
+};
+__host__ __device__ constexpr RouteLds route_lds(int T, int E, int k) {
+  RouteLds L{};
+  int o = 0;
+  auto take = [&](int words) {
+    o = (o + 3) & ~3;
+    const int at = o;
+    o += words;
+    return at;
+  };
+  L.tabs = take(3 * ((2 * E + 3) & ~3));
+  L.ev = take(T * ((E + 31) & ~31));
+  L.ridx = take(T * k);
+  L.rw = take(T * (k + 1));
+  L.keys = take(T * k);
+  L.sorted = take(T * k);
+  L.cnt = take(2 * kRouteWaves);
+  L.total = (o + 3) & ~3;
+  return L;
+}
+__host__ inline int route_grid(int T, int hidden, bool gate) {
+  return 1 + (T * (hidden / kQK) + 4 * kRouteWaves - 1) / (4 * kRouteWaves) + gate;
+}
+
+// PL: experts per lane (n_expert <= 64 PL)
+template <int PL>
+__device__ __forceinline__ void route_body(const LayerArgs& a, uint32_t* dyn) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int T = a.T, k = a.k, E = a.n_expert, stride = k + 1, R = T * k;
+  if (blockIdx.x > 0) {
+    const int nxb = T * (a.hidden / kQK);
+    const int b = 4 * (kRouteWaves * (static_cast<int>(blockIdx.x) - 1) + wave) + (lane >> 4);
+    if (4 * kRouteWaves * (static_cast<int>(blockIdx.x) - 1) >= nxb) {
+      shared_gate_tokens(a, tid, kRouteThreads / 32);
+      return;
+    }
+    float v[16];
+    x_load16(a, b < nxb ? b : 0, lane, v);
+    x_row16_lds(a, v, a.xq + static_cast<long long>(b < nxb ? b : 0) * kXStride, b < nxb, lane);
+    return;
+  }
+  const RouteLds L = route_lds(T, E, k);
+  const int e32 = (E + 31) & ~31, tab_words = (2 * E + 3) & ~3;
+  int* ridx = reinterpret_cast<int*>(dyn + L.ridx);
+  float* rw = reinterpret_cast<float*>(dyn + L.rw);
+  int* keys = reinterpret_cast<int*>(dyn + L.keys);
+  int* sorted = reinterpret_cast<int*>(dyn + L.sorted);
+  int* cnt = reinterpret_cast<int*>(dyn + L.cnt);  // per wave: group starts, valid routes
+  // the pointer tables into LDS, by the last waves (the tokens take the first)
+  auto copy_table = [&](const sg_block_q4k* const* tab, int m) {
+    uint32_t* dst = dyn + L.tabs + m * tab_words;
+    const char* src = reinterpret_cast<const char*>(tab);
+    dma_range([&](int c) { return src + 16 * c; }, E / 2, dst, lane);
+    if ((E & 1) && lane == 0)  // odd table length: the last pointer by a plain load
+      reinterpret_cast<unsigned long long*>(dst)[E - 1] =
+          reinterpret_cast<unsigned long long>(tab[E - 1]);
+  };
+  if (wave == kRouteWaves - 3) copy_table(a.tab_gate, 0);
+  else if (wave == kRouteWaves - 2) copy_table(a.tab_up, 1);
+  else if (wave == kRouteWaves - 1) copy_table(a.tab_down, 2);
+  if (a.logits) {
+    if (wave < T)
+      router_wave<PL>(a.logits + static_cast<long long>(wave) * E, E, k, a.shared_w,
+                      ridx + wave * k, rw + wave * stride,
+                      reinterpret_cast<float*>(dyn + L.ev) + wave * e32, lane);
+  } else {
+    for (int i = tid; i < R; i += kRouteThreads) ridx[i] = a.idx[(i / k) * stride + (i % k)];
+    for (int i = tid; i < T * stride; i += kRouteThreads) rw[i] = a.weight[i];
+  }
+  bar();
+  // keys (expert, route), below 2^20; an invalid id sorts last and is left out
+  constexpr int kInvalid = 1024 << 9;
+  int key = 0x7FFFFFFF;
+  if (tid < R) {
+    const int e = ridx[tid];
+    key = (e >= 0 && e < E ? e << 9 : kInvalid) + tid;
+    keys[tid] = key;
+  }
+  bar();
+  if (tid < R) {
+    int rank = 0;
+    for (int j0 = 0; j0 < R; j0 += 4) {  // (a comparison is the sign bit of a difference)
+      const int4 v = *reinterpret_cast<const int4*>(keys + j0);
+      const int kv[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (j0 + u < R)
+          rank += static_cast<int>(__builtin_amdgcn_ubfe(static_cast<unsigned>(kv[u] - key), 31, 1));
+    }
+    sorted[rank] = key;
+  }
+  bar();
+  const int sk = tid < R ? sorted[tid] : kInvalid;  // thread r: the r-th entry
+  const int se = sk >> 9, si = sk & 511;
+  const bool valid = sk < kInvalid;
+  const bool first = valid && (tid == 0 || (sorted[tid - 1] >> 9) != se);
+  const uint64_t fm = __ballot(first), vm = __ballot(valid);
+  if (lane == 0) {
+    cnt[wave] = __popcll(fm);
+    cnt[kRouteWaves + wave] = __popcll(vm);
+  }
+  wait_vm();  // the pointer tables
+  bar();
+  int grp = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(fm >> 32),
+                                      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(fm), 0));
+  int nf = 0, nv = 0;
+#pragma unroll
+  for (int w = 0; w < kRouteWaves; ++w) {
+    const int c = cnt[w];
+    grp += w < wave ? c : 0;
+    nf += c;
+    nv += cnt[kRouteWaves + w];
+  }
+  const int gbase = a.has_shared ? (T + a.split - 1) / a.split : 0, ebase = a.has_shared ? T : 0;
+  auto put_group = [&](int g, int off, unsigned long long gp, unsigned long long up,
+                       unsigned long long dp) {
+    a.plan.off[g] = off;
+    const bool present = gp && up;
+    a.plan.wdown[g] = present ? dp : 0ull;
+    a.plan.wgate[g] = present ? gp : 0ull;
+    a.plan.wup[g] = present ? up : 0ull;
+  };
+  const unsigned long long* tabg = reinterpret_cast<const unsigned long long*>(dyn + L.tabs);
+  const unsigned long long* tabu = reinterpret_cast<const unsigned long long*>(dyn + L.tabs + tab_words);
+  const unsigned long long* tabd =
+      reinterpret_cast<const unsigned long long*>(dyn + L.tabs + 2 * tab_words);
+  if (valid) {
+    a.plan.tok[ebase + tid] = si / k;
+    a.plan.slot[ebase + tid] = si % k;
+    if (first) put_group(gbase + grp, ebase + tid, tabg[se], tabu[se], tabd[se]);
+  }
+  if (tid < gbase)
+    put_group(tid, tid * a.split, reinterpret_cast<unsigned long long>(a.sh_gate),
+              reinterpret_cast<unsigned long long>(a.sh_up),
+              reinterpret_cast<unsigned long long>(a.sh_down));
+  if (tid < ebase) {
+    a.plan.tok[tid] = tid;
+    a.plan.slot[tid] = k;
+  }
+  if (tid == 0) {
+    a.plan.off[gbase + nf] = ebase + nv;
+    a.plan.meta[0] = gbase + nf;
+    a.plan.meta[1] = a.has_shared;
+    a.plan.meta[2] = nv;
+  }
+  for (int i = tid; i < T * stride; i += kRouteThreads) {
+    const int t = i / stride, q = i - t * stride;
+    bool bad = false;  // bounds-kill: a row with an invalid id loses all its weights
+    for (int kk = 0; kk < k; ++kk) {
+      const int e = ridx[t * k + kk];
+      bad |= e < 0 || e >= E;
+    }
+    a.weight[i] = bad ? 0.f : rw[i];
+    if (a.logits && q < k) a.idx[i] = ridx[t * k + q];
+  }
+}
+
+// kOne: the one-token kernel (routing, gate/up and SiLU in one launch, EPT
+// experts per thread); otherwise the routing launch of several tokens (EPT
+// experts per lane).
 template <int EPT, int NBH, bool kOne = false, int kShapeT = 0, bool kSh = false, int kIo = 0>
-__global__ void __launch_bounds__(256) layer_front_kernel(LayerArgs args) {
+__global__ void __launch_bounds__(kOne ? kFrontThreads : kRouteThreads)
+layer_front_kernel(LayerArgs args) {
   LayerArgs a = args;
   apply_shape<kShapeT, kSh, kIo>(a);
-  __shared__ __attribute__((aligned(16))) uint32_t wbuf[4][64 * 36];
   extern __shared__ __attribute__((aligned(16))) uint32_t dyn[];
-  // Row y of the grid runs group g.  With a shared expert its row comes
-  // after the routed ones: workgroups are placed on CUs in grid order, so the
-  // routed workgroups (the long routing chain) each get a CU of their own
-  // and the shared expert's (no routing, done early) double up.
-  // (one token only: the grid is then about one workgroup per CU; with more
-  // tokens the shared expert's row stays first so it is not the tail)
-  const int y = blockIdx.y;
-  const int g = !kOne && a.publish_only
-                    ? a.gmax
-                    : ((!kOne && a.T != 1) || !a.has_shared || y >= a.gmax
-                           ? y
-                           : (y + 1 == a.gmax ? 0 : y + 1));
-  front_body<EPT, NBH, kOne>(a, blockIdx.x, g, wbuf, dyn);
+  if constexpr (kOne) {
+    __shared__ __attribute__((aligned(16))) uint32_t wbuf[4][64 * 36];
+    // Row y of the grid runs group g.  With a shared expert its row comes
+    // after the routed ones: workgroups are placed on CUs in grid order, so the
+    // routed workgroups (the long routing chain) each get a CU of their own
+    // and the shared expert's (no routing, done early) double up.
+    const int y = blockIdx.y;
+    const int g = !a.has_shared || y >= a.gmax ? y : (y + 1 == a.gmax ? 0 : y + 1);
+    front_body<EPT, NBH>(a, blockIdx.x, g, wbuf, dyn);
+  } else {
+    route_body<EPT>(a, dyn);
+  }
 }
 
 // Gate/up + SiLU of one (row chunk, group) from the plan the routing launch
@@ -1624,7 +1567,34 @@ layer_gateup_kernel(LayerArgs args) {
   gateup_group(present, row0, nrw, nbh, lpr, wbuf[wave], &wbuf[0][0], x0, a.xq,
                [&](int j, int& t, int& sl) { t = etok[j0 + j]; sl = eslot[j0 + j]; }, n, stride,
                a.n_ff, a.h, lane, wave, a.out16 != nullptr);
-  if (g == 0 && a.has_shared && a.sh_gate_w && bx == 0) shared_gate_tokens(a, tid);
+}
+
+// ---- Q8_K of h (many tokens) -------------------------------------------------------------
+// Every back workgroup reads every (token, slot) h row as Q8_K.  Quantizing
+// them there costs each of the 256 workgroups 0.33 us for eight blocks, so from
+// kHqBlocks blocks on one launch does it, in place: a wave reads four 256-value
+// blocks whole before it writes, and block e's Q8_K (kXStride words, the LDS
+// layout) takes the head of its 1024 B.  The line, per layer, in the back
+// kernel / by the launch: hidden 2048, 36 blocks 26.2 / 26.7 us, 54 29.7 / 29.9,
+// 90 39.1 / 37.2, 288 79.6 / 65.6; hidden 1280, 48 blocks 37.9 / 35.3.
+constexpr int kHqBlocks = 48;
+static_assert(kShapeWindow * (kShapeK + 1) * (kShapeFf / kQK) >= kHqBlocks,
+              "the window's instances take h quantized");
+__global__ void __launch_bounds__(256) layer_hq_kernel(float* h, int n_blocks) {
+  const int lane = threadIdx.x & 63;
+  const int b = blockIdx.x * 16 + 4 * (threadIdx.x >> 6) + (lane >> 4);
+  float* hb = h + static_cast<long long>(b < n_blocks ? b : n_blocks - 1) * kQK;
+  float v[16];
+#pragma unroll
+  for (int i = 0; i < 16; i += 4) {
+    const float4 f = *reinterpret_cast<const float4*>(hb + 16 * (lane & 15) + i);
+    v[i] = f.x;
+    v[i + 1] = f.y;
+    v[i + 2] = f.z;
+    v[i + 3] = f.w;
+  }
+  // (the block's maximum needs every lane's values: no store comes before the loads)
+  quantize_row16_lds(v, reinterpret_cast<uint32_t*>(hb), b < n_blocks, lane);
 }
 
 // ---- back kernel ------------------------------------------------------------------------
@@ -1632,7 +1602,8 @@ layer_gateup_kernel(LayerArgs args) {
 // shape allows).  A wave packs `gpw` groups side by side - lane = (group,
 // row, super-block) - and streams their down rows for the chunk into its LDS
 // buffer while all eight waves quantize every (token, slot) h row to Q8_K in
-// LDS (h was loaded at kernel start, beside the plan).  The slot outputs of
+// LDS (h was loaded at kernel start, beside the plan; with many tokens it is
+// quantized already and copied).  The slot outputs of
 // the chunk go to LDS; then the workgroup combines
 // out = residual + sum_kk fma(w_kk, y_kk) in slot order.
 constexpr int kBackWaves = 8;                    // waves per back workgroup
@@ -1704,6 +1675,50 @@ __device__ __forceinline__ void back_quantize_h(const LayerArgs& a, uint32_t* hq
   }
 }
 
+// The combine of one chunk, from the slot outputs in ys (complete and visible).
+__device__ __forceinline__ void back_combine(const LayerArgs& a, const BackLds& L, const uint32_t* bd,
+                                             int row0, int nr, float res0, int rows) {
+  const int tid = threadIdx.x, T = a.T, k = a.k, stride = k + 1;
+  const float* ys = reinterpret_cast<const float*>(bd + L.ys);
+  const float* wt = reinterpret_cast<const float*>(bd + L.wt);
+  const float* sgl = reinterpret_cast<const float*>(bd + L.sg);
+  const int n_out = T * nr;
+  // out = residual + sum over slots 0..k of fma(w, y) in slot order.  A slot
+  // whose id was invalid (bounds-killed), whose expert is absent, or the
+  // shared slot without a shared expert has no plan entry, so its y is the
+  // 0 the prologue stored.
+  for (int qo = tid; qo < n_out; qo += kBackThreads) {
+    const int t = qo / nr, r = qo - t * nr;
+    const long long o = static_cast<long long>(t) * a.hidden + row0 + r;
+    float acc = qo == tid ? res0
+                          : (a.residual ? a.residual[o] : (a.res16 ? f16v(a.res16[o]) : 0.f));
+    // the shared slot's output scaled by its gate first (1.0 without a
+    // gate, which leaves it unchanged), as sigmoid_gate_scalar_batched_f16
+    // does before the combine (session.cpp:2904-2909)
+    const float gs = sgl[t];
+    for (int k0 = 0; k0 <= k; k0 += 16) {  // gather 16 slots, then the ordered fma chain
+      float yv[16], wv[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const int i = t * stride + (k0 + u <= k ? k0 + u : k);
+        yv[u] = ys[i * rows + r];
+        wv[u] = wt[i];
+        if (a.out16) {  // fp16 slot outputs; the shared one gated on its fp16 value
+          yv[u] = f16v(f16b(yv[u]));
+          if (k0 + u == k) yv[u] = f16v(f16b(yv[u] * gs));
+        } else if (k0 + u == k) {
+          yv[u] *= gs;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+        if (k0 + u <= k) acc = __builtin_fmaf(wv[u], yv[u], acc);
+    }
+    if (a.out16) a.out16[o] = f16b(acc);
+    else a.out[o] = acc;
+  }
+}
+
 // The down rows, Q8_K of h and combine of one chunk of `rows` output rows,
 // with the plan in LDS (off, wdown, tok, slot, wt, meta).  Wave w
 // quantizes h blocks w + 8j; hpre[j] holds the lane's 4 values of block
@@ -1728,11 +1743,8 @@ __device__ __forceinline__ void back_core(const LayerArgs& a, const BackLds& L, 
   const unsigned long long* wdown = reinterpret_cast<const unsigned long long*>(bd + L.wdown);
   const int* tok = reinterpret_cast<const int*>(bd + L.tok);
   const int* slot = reinterpret_cast<const int*>(bd + L.slot);
-  const float* wt = reinterpret_cast<const float*>(bd + L.wt);
-  const float* sgl = reinterpret_cast<const float*>(bd + L.sg);
   const int* meta = reinterpret_cast<const int*>(bd + L.meta);
   const int nq = T * stride * nbf;
-  const int n_out = T * nr;
   const int G = __builtin_amdgcn_readfirstlane(meta[0]);
   const int gwords = rows * nbf * 36;  // one group's rows in the buffer
   uint32_t* buf = wbuf[wave];
@@ -1842,7 +1854,30 @@ __device__ __forceinline__ void back_core(const LayerArgs& a, const BackLds& L, 
       const float acc = blk2 == 1 ? prev2 + bsum : acc0;
       if (ok && has && hf == 1 && blk2 == 1 && rr2 < nr) ys[hs * rows + rr2] = present ? acc : 0.f;
     }
-  } else
+    bar();
+    back_combine(a, L, bd, row0, nr, res0, rows);
+    return;
+  }
+  // down rows of this wave's gpw groups gb + wave * gpw .. as one run of 16-B
+  // chunks: chunk c = group c / cpg, chunk c % cpg of the group's rows; LDS
+  // destination buf + 4c (group qq at buf + qq * gwords).  At most 9 copy
+  // instructions, no loop over groups.
+  auto issue = [&](int gb) {
+    const int cpg = gwords / 4;       // chunks per group slot
+    const int cval = nr * nbf * 9;    // chunks present (nr < rows at the edge)
+    const uint32_t inv = ((1u << 20) + cpg - 1) / cpg;  // c / cpg exact for c < 576
+    const long long roff = static_cast<long long>(row0) * nbf * kQ4Bytes;
+#pragma unroll 1
+    for (int i = 0; 64 * i < gpw * cpg; ++i) {
+      const int c = lane + 64 * i;
+      const int qq = static_cast<int>((static_cast<uint32_t>(c) * inv) >> 20);
+      const int w = c - qq * cpg;
+      const int gq = gb + wave * gpw + qq;
+      const unsigned long long wd = qq < gpw && gq < G && wave < nbw ? wdown[gq] : 0ull;
+      if (wd && w < cval)
+        dma16_stream(buf + 256 * i, reinterpret_cast<const char*>(wd) + roff + 16 * w);
+    }
+  };
   for (int gb = 0; gb < G; gb += nbw * gpw) {
     if (spread) {
       // every group's down rows as one run of 16-B chunks over all the
@@ -1864,32 +1899,12 @@ __device__ __forceinline__ void back_core(const LayerArgs& a, const BackLds& L, 
                 (lds_void_p)(wbuf[0] + 256 * t), 16, 0, kNt);
         }
       }
-    } else {
-      // down rows of this wave's gpw groups as one run of 16-B chunks: chunk
-      // c = group c / cpg, chunk c % cpg of the group's rows; LDS destination
-      // buf + 4c (group qq at buf + qq * gwords).  At most 9 copy
-      // instructions, no loop over groups.
-      const int cpg = gwords / 4;       // chunks per group slot
-      const int cval = nr * nbf * 9;    // chunks present (nr < rows at the edge)
-      const uint32_t inv = ((1u << 20) + cpg - 1) / cpg;  // c / cpg exact for c < 576
-      const long long roff = static_cast<long long>(row0) * nbf * kQ4Bytes;
-#pragma unroll
-      for (int i = 0; i < 9; ++i) {
-        const int c = lane + 64 * i;
-        if (64 * i >= gpw * cpg) break;
-        const int qq = static_cast<int>((static_cast<uint32_t>(c) * inv) >> 20);
-        const int w = c - qq * cpg;
-        const int gq = gb + wave * gpw + qq;
-        const unsigned long long wd = qq < gpw && gq < G && wave < nbw ? wdown[gq] : 0ull;
-        if (wd && w < cval)
-          __builtin_amdgcn_global_load_lds(
-              (glb_void_p)(reinterpret_cast<const char*>(wd) + roff + 16 * w),
-              (lds_void_p)(buf + 256 * i), 16, 0, kNt);
-      }
+    } else if (gb == 0) {
+      issue(0);
     }
     if (gb == 0 && !pre) {  // Q8_K of every (token, slot) h row while the rows stream in
-      back_quantize_h<HS>(a, hq, hpre, nq, wave, lane);
-      if (spread) wait_vm();  // this wave's share of the copies
+      if (!a.hq_pre) back_quantize_h<HS>(a, hq, hpre, nq, wave, lane);
+      if (spread || a.hq_pre) wait_vm();  // this wave's share of the copies
       bar();
     }
     wait_vm();
@@ -1903,6 +1918,9 @@ __device__ __forceinline__ void back_core(const LayerArgs& a, const BackLds& L, 
       read_block_lds(buf + q * gwords + 36 * (rr * nbf + blk), w36);
       sm8 = unpack_scales(w36[1], w36[2], w36[3]);
     }
+    // the next pass's rows stream in during this one's dots
+    wait_lds();
+    if (!spread && gb + nbw * gpw < G) issue(gb + nbw * gpw);
     // entries of the group, clamped to the plan's capacity (a plan is only
     // ever read here, never trusted to bound a loop)
     const int jb = has ? min(max(off[gq], 0), a.emax) : 0;
@@ -1923,43 +1941,9 @@ __device__ __forceinline__ void back_core(const LayerArgs& a, const BackLds& L, 
       const float acc = row_sum_last(s, blk, nbf);
       if (ok && blk == nbf - 1 && rr < nr) ys[hs * rows + rr] = present ? acc : 0.f;
     }
-    wait_lds();
   }
   bar();
-  // out = residual + sum over slots 0..k of fma(w, y) in slot order.  A slot
-  // whose id was invalid (bounds-killed), whose expert is absent, or the
-  // shared slot without a shared expert has no plan entry, so its y is the
-  // 0 the prologue stored.
-  for (int qo = tid; qo < n_out; qo += kBackThreads) {
-    const int t = qo / nr, r = qo - t * nr;
-    const long long o = static_cast<long long>(t) * a.hidden + row0 + r;
-    float acc = qo == tid ? res0
-                          : (a.residual ? a.residual[o] : (a.res16 ? f16v(a.res16[o]) : 0.f));
-    // the shared slot's output scaled by its gate first (1.0 without a
-    // gate, which leaves it unchanged), as sigmoid_gate_scalar_batched_f16
-    // does before the combine (session.cpp:2904-2909)
-    const float gs = sgl[t];
-    for (int k0 = 0; k0 <= k; k0 += 16) {  // gather 16 slots, then the ordered fma chain
-      float yv[16], wv[16];
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        const int i = t * stride + (k0 + u <= k ? k0 + u : k);
-        yv[u] = ys[i * rows + r];
-        wv[u] = wt[i];
-        if (a.out16) {  // fp16 slot outputs; the shared one gated on its fp16 value
-          yv[u] = f16v(f16b(yv[u]));
-          if (k0 + u == k) yv[u] = f16v(f16b(yv[u] * gs));
-        } else if (k0 + u == k) {
-          yv[u] *= gs;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 16; ++u)
-        if (k0 + u <= k) acc = __builtin_fmaf(wv[u], yv[u], acc);
-    }
-    if (a.out16) a.out16[o] = f16b(acc);
-    else a.out[o] = acc;
-  }
+  back_combine(a, L, bd, row0, nr, res0, rows);
 }
 
 // residual of the first combine pass (qo = tid), loaded early
@@ -2002,9 +1986,19 @@ __global__ void __launch_bounds__(kBackThreads) layer_back_kernel(LayerArgs args
   // loads that do not depend on the plan: this wave's first HS h
   // blocks (block wave + 8j of the (token, slot) rows) and the residual
   const int nq = T * stride * nbf;
-  constexpr int HS = kShapeT == kShapeWindow ? 9 : kBackHSlots;  // the window: every block
+  constexpr int HS = kBackHSlots;
   float hpre[HS][4];
-  if (wave < nq) {
+  if (a.hq_pre) {  // quantized already: 320 of each block's 1024 B into LDS
+    const char* src = reinterpret_cast<const char*>(a.h);
+    uint32_t* hq = dyn + L.hq;
+    constexpr int kCpb = kXStride / 4;  // 16-B chunks per block
+    for (int c0 = 64 * wave; c0 < nq * kCpb; c0 += 64 * kBackWaves) {
+      const int c = c0 + lane, e = c / kCpb;
+      if (c < nq * kCpb)
+        __builtin_amdgcn_global_load_lds((glb_void_p)(src + 1024 * e + 16 * (c - e * kCpb)),
+                                         (lds_void_p)(hq + 4 * c0), 16, 0, 0);
+    }
+  } else if (wave < nq) {
 #pragma unroll
     for (int j = 0; j < HS; ++j) {
       const int e0 = wave + kBackWaves * j;
@@ -2118,11 +2112,24 @@ __global__ void __launch_bounds__(kBackThreads) layer_back_kernel(LayerArgs args
   }
   for (int i = tid; i < T * stride * rows; i += kBackThreads) ys[i] = 0.f;
   if (pre) {
-    back_quantize_h<HS>(a, dyn + L.hq, hpre, nq, wave, lane);
+    if (!a.hq_pre) back_quantize_h<HS>(a, dyn + L.hq, hpre, nq, wave, lane);
     wait_vm();  // this wave's copies, visible to all after the barrier
   }
   bar();
   back_core<NBF, ROWS, HS>(a, L, dyn, wbuf, row0, nr, res0, hpre, pre);
+}
+
+// The layer's limit on shapes: every token's staged x, the pointer tables and
+// the routing arrays within one workgroup's LDS beside four weight buffers.
+static bool layer_lds_refused(int T, int nbh, int E, int k) {
+  const int teams = T == 1 ? 1 : (T == 2 ? 2 : 4), m = k + 1, e32 = (E + 31) & ~31;
+  const int ncp = (4 / teams * m + 3) & ~3, gmax = (T * k < E ? T * k : E) + 1;
+  const int words[] = {T * nbh * kXStride, 2 * E, 2 * E, 2 * E, teams * e32, 4 * e32,
+                       teams * ncp * 2, teams * m * 2, teams * 4, teams, T * m, T * k, T * m, T * k,
+                       T * k, gmax + 1, gmax, T * m, T * m, 8 + T * k, 768};
+  int o = 0;
+  for (int w : words) o = ((o + 3) & ~3) + w;
+  return static_cast<size_t>(o) * 4 + 4 * 64 * 36 * 4 > 160 * 1024;
 }
 
 static void back_geometry(int hidden, int n_ff, int& rows, int& lrow) {
@@ -2192,7 +2199,7 @@ extern "C" {
 
 size_t sg_moe_layer_workspace_bytes(int n_tokens, int hidden, int n_ff, int n_expert, int k) {
   if (n_tokens <= 0 || hidden <= 0 || n_ff <= 0 || n_expert <= 0 || k <= 0) return 0;
-  return layer_ws(n_tokens, hidden, n_ff, n_expert, k).total;
+  return layer_ws(n_tokens, hidden, n_ff, n_expert, k, kShSplit).total;
 }
 
 int sg_moe_layer_stages(const sg_block_q4k* const* tab_gate, const sg_block_q4k* const* tab_up,
@@ -2261,18 +2268,32 @@ static int layer_launch(const sg_block_q4k* const* tab_gate, const sg_block_q4k*
                      n_expert, kLMaxExperts);
   int rows = 1, lrow = 64;
   back_geometry(hidden, n_ff, rows, lrow);
-  const LayerWs ws = layer_ws(n_tokens, hidden, n_ff, n_expert, k);
+  // the back kernel's down-row buffers: one per wave when they fit, else four
+  const size_t buf_b = 64 * 36 * 4;
+  // The shared expert in groups of kShSplit tokens, or in one where the
+  // workspace or the back kernel's LDS has no room for their few plan entries
+  int split = kShSplit;
+  LayerWs ws{};
+  size_t lds_b = 0;
+  for (;; split = n_tokens) {
+    ws = layer_ws(n_tokens, hidden, n_ff, n_expert, k, split);
+    lds_b = static_cast<size_t>(back_lds(n_tokens, k, n_ff, rows, ws.gmax, ws.emax).total) * 4;
+    if (split >= n_tokens ||
+        (workspace_bytes >= ws.total && lds_b + 4 * buf_b <= 160 * 1024)) break;
+  }
   if (workspace_bytes < ws.total)
     return set_error(SG_ERR_INVALID_ARGUMENT, "%s: workspace %zu < %zu bytes", nm,
                      workspace_bytes, ws.total);
+  // one token: the front kernel's LDS; several: the routing launch's, and the
+  // gate/up launch's (the first entry's x, then the entries)
+  const bool one = n_tokens == 1;
   const size_t lds_f =
-      static_cast<size_t>(front_lds(n_tokens, hidden / kQK, n_expert, k, true).total) * 4;
-  const size_t lds_b =
-      static_cast<size_t>(back_lds(n_tokens, k, n_ff, rows, ws.gmax, ws.emax).total) * 4;
-  // the back kernel's down-row buffers: one per wave when they fit, else four
-  const size_t buf_b = 64 * 36 * 4;
+      static_cast<size_t>(one ? front_lds(hidden / kQK, n_expert, k, true).total
+                              : route_lds(n_tokens, n_expert, k).total) * 4;
+  const size_t lds_g = static_cast<size_t>((((hidden / kQK) * kXStride + 3) & ~3) + 2 * ws.emax) * 4;
   const int back_bufs = lds_b + kBackWaves * buf_b <= 160 * 1024 ? kBackWaves : 4;
-  if (lds_f + 4 * buf_b > 160 * 1024 || lds_b + back_bufs * buf_b > 160 * 1024)
+  if (layer_lds_refused(n_tokens, hidden / kQK, n_expert, k) ||
+      lds_b + back_bufs * buf_b > 160 * 1024 || (!one && lds_g + 4 * buf_b > 160 * 1024))
     return set_error(SG_ERR_UNSUPPORTED, "%s: this shape needs more LDS than a workgroup has",
                      nm);
   unsigned char* base = static_cast<unsigned char*>(workspace);
@@ -2297,7 +2318,6 @@ static int layer_launch(const sg_block_q4k* const* tab_gate, const sg_block_q4k*
   a.idx = idx;
   a.weight = weight;
   a.plan = LayerPlan{reinterpret_cast<int*>(base + ws.meta), reinterpret_cast<int*>(base + ws.off),
-                     reinterpret_cast<int*>(base + ws.expert),
                      reinterpret_cast<int*>(base + ws.tok), reinterpret_cast<int*>(base + ws.slot),
                      reinterpret_cast<unsigned long long*>(base + ws.wdown),
                      reinterpret_cast<unsigned long long*>(base + ws.wgate),
@@ -2317,61 +2337,52 @@ static int layer_launch(const sg_block_q4k* const* tab_gate, const sg_block_q4k*
   a.back_rows = rows;
   a.back_lrow = lrow;
   a.back_bufs = back_bufs;
+  a.split = split;
+  const int nq = n_tokens * (k + 1) * (n_ff / kQK);  // h blocks
+  a.hq_pre = !one && nq >= kHqBlocks;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int rows_wg = 4 * (32 / pow2_ceil(hidden / kQK));
-  const FrontLds fl = front_lds(n_tokens, hidden / kQK, n_expert, k, true);
-  a.front_routed = fl;
-  a.front_shared = front_lds(n_tokens, hidden / kQK, n_expert, k, false);
-  // several tokens: routing launch (the publisher alone), then the gate/up
-  // launch reading its plan; one token: one fused launch whose compute
-  // workgroups route speculatively beside their weight stream
-  // the gate/up launch: the first entry's x, then the entries
-  const size_t lds_g = static_cast<size_t>((((hidden / kQK) * kXStride + 3) & ~3) + 2 * ws.emax) * 4;
-  a.publish_only = n_tokens > 1;
-  if (a.publish_only && lds_g + 4 * buf_b > 160 * 1024)
-    return set_error(SG_ERR_UNSUPPORTED, "%s: this shape needs more LDS than a workgroup has",
-                     nm);
+  a.front_routed = front_lds(hidden / kQK, n_expert, k, true);
+  a.front_shared = front_lds(hidden / kQK, n_expert, k, false);
+  // One token: one launch whose compute workgroups route speculatively beside
+  // their weight stream (y < gmax: compute workgroups of group y; y == gmax:
+  // the publisher).  Several: the routing launch, the gate/up launch reading
+  // its plan, and with many tokens the Q8_K of h.
+  const bool window = is_shape(n_tokens, hidden, n_ff, n_expert, k, kShapeWindow) && a.has_shared;
   if (stages & 1) {
-    // y < gmax: compute workgroups of group y; y == gmax: the publisher
-    const dim3 grid = a.publish_only ? dim3(1, 1)
-                                     : dim3((n_ff + rows_wg - 1) / rows_wg, ws.gmax + 1);
-    if (is_shape(n_tokens, hidden, n_ff, n_expert, k, 1) && a.has_shared) {  // the model shape
-      if (f32io)
-        hipLaunchKernelGGL((layer_front_kernel<1, 8, true, 1, true, 1>), grid, dim3(256), lds_f, s, a);
-      else
-        hipLaunchKernelGGL((layer_front_kernel<1, 8, true, 1, true, 2>), grid, dim3(256), lds_f, s, a);
-    } else if (is_shape(n_tokens, hidden, n_ff, n_expert, k, 1)) {
-      if (f32io)
-        hipLaunchKernelGGL((layer_front_kernel<1, 8, true, 1, false, 1>), grid, dim3(256), lds_f, s, a);
-      else
-        hipLaunchKernelGGL((layer_front_kernel<1, 8, true, 1, false, 2>), grid, dim3(256), lds_f, s, a);
-    } else if (is_shape(n_tokens, hidden, n_ff, n_expert, k, kShapeWindow) && a.has_shared) {
-      if (f32io)  // its verify window
-        hipLaunchKernelGGL((layer_front_kernel<4, 8, false, kShapeWindow, true, 1>), grid, dim3(256),
-                           lds_f, s, a);
-      else
-        hipLaunchKernelGGL((layer_front_kernel<4, 8, false, kShapeWindow, true, 2>), grid, dim3(256),
-                           lds_f, s, a);
+    auto front = [&](auto kern) {
+      hipLaunchKernelGGL(kern, one ? dim3((n_ff + rows_wg - 1) / rows_wg, ws.gmax + 1)
+                                   : dim3(route_grid(n_tokens, hidden, a.sh_gate_w != nullptr)),
+                         dim3(one ? kFrontThreads : kRouteThreads), lds_f, s, a);
+    };
+    if (is_shape(n_tokens, hidden, n_ff, n_expert, k, 1)) {  // the model shape
+      if (a.has_shared && f32io) front(layer_front_kernel<1, 8, true, 1, true, 1>);
+      else if (a.has_shared) front(layer_front_kernel<1, 8, true, 1, true, 2>);
+      else if (f32io) front(layer_front_kernel<1, 8, true, 1, false, 1>);
+      else front(layer_front_kernel<1, 8, true, 1, false, 2>);
+    } else if (one) {
+      const int ept = a.front_routed.ept;
+      if (ept <= 1 && hidden / kQK == 8) front(layer_front_kernel<1, 8, true>);
+      else if (ept <= 1) front(layer_front_kernel<1, 0, true>);
+      else if (ept <= 2) front(layer_front_kernel<2, 0, true>);
+      else front(layer_front_kernel<4, 0, true>);
+    } else if (window) {  // its verify window
+      if (f32io) front(layer_front_kernel<4, 8, false, kShapeWindow, true, 1>);
+      else front(layer_front_kernel<4, 8, false, kShapeWindow, true, 2>);
+    } else {
+      if (n_expert <= 64) front(layer_front_kernel<1, 0>);
+      else if (n_expert <= 128) front(layer_front_kernel<2, 0>);
+      else if (n_expert <= 256) front(layer_front_kernel<4, 0>);
+      else if (n_expert <= 512) front(layer_front_kernel<8, 0>);
+      else front(layer_front_kernel<16, 0>);
     }
-    else if (fl.ept <= 1 && hidden / kQK == 8 && n_tokens == 1)  // one-token decode, hidden 2048
-      hipLaunchKernelGGL((layer_front_kernel<1, 8, true>), grid, dim3(256), lds_f, s, a);
-    else if (fl.ept <= 1 && hidden / kQK == 8)  // the decode shape, compiled for hidden 2048
-      hipLaunchKernelGGL((layer_front_kernel<1, 8>), grid, dim3(256), lds_f, s, a);
-    else if (fl.ept <= 1)
-      hipLaunchKernelGGL((layer_front_kernel<1, 0>), grid, dim3(256), lds_f, s, a);
-    else if (fl.ept <= 2)
-      hipLaunchKernelGGL((layer_front_kernel<2, 0>), grid, dim3(256), lds_f, s, a);
-    else if (fl.ept <= 4)
-      hipLaunchKernelGGL((layer_front_kernel<4, 0>), grid, dim3(256), lds_f, s, a);
-    else
-      hipLaunchKernelGGL((layer_front_kernel<kMaxEpt, 0>), grid, dim3(256), lds_f, s, a);
     if (int st = check_launch("sg_moe_layer/front")) return st;
-    if (a.publish_only) {
+    if (!one) {
       const dim3 gg((n_ff + rows_wg - 1) / rows_wg, ws.gmax);
-      if (is_shape(n_tokens, hidden, n_ff, n_expert, k, kShapeWindow) && a.has_shared && f32io)
+      if (window && f32io)
         hipLaunchKernelGGL((layer_gateup_kernel<8, kShapeWindow, true, 1>), gg, dim3(256), lds_g, s,
                            a);
-      else if (is_shape(n_tokens, hidden, n_ff, n_expert, k, kShapeWindow) && a.has_shared)
+      else if (window)
         hipLaunchKernelGGL((layer_gateup_kernel<8, kShapeWindow, true, 2>), gg, dim3(256), lds_g, s,
                            a);
       else if (hidden / kQK == 8)
@@ -2379,6 +2390,10 @@ static int layer_launch(const sg_block_q4k* const* tab_gate, const sg_block_q4k*
       else
         hipLaunchKernelGGL((layer_gateup_kernel<0>), gg, dim3(256), lds_g, s, a);
       if (int st = check_launch("sg_moe_layer/gateup")) return st;
+      if (a.hq_pre) {
+        hipLaunchKernelGGL(layer_hq_kernel, dim3((nq + 15) / 16), dim3(256), 0, s, a.h, nq);
+        if (int st = check_launch("sg_moe_layer/quantize_h")) return st;
+      }
     }
   }
   if (stages & 2) {
@@ -2397,8 +2412,7 @@ static int layer_launch(const sg_block_q4k* const* tab_gate, const sg_block_q4k*
         hipLaunchKernelGGL((layer_back_kernel<2, 8, 1, false, 1>), gb, dim3(kBackThreads), lds_bb, s, a);
       else
         hipLaunchKernelGGL((layer_back_kernel<2, 8, 1, false, 2>), gb, dim3(kBackThreads), lds_bb, s, a);
-    } else if (geo && is_shape(n_tokens, hidden, n_ff, n_expert, k, kShapeWindow) &&
-               a.has_shared) {  // its verify window
+    } else if (geo && window) {  // its verify window
       if (f32io)
         hipLaunchKernelGGL((layer_back_kernel<2, 8, kShapeWindow, true, 1>), gb, dim3(kBackThreads),
                            lds_bb, s, a);
@@ -2441,7 +2455,11 @@ int sg_moe_layer_noalloc(const sg_block_q4k* const* tab_gate, const sg_block_q4k
                          int n_tokens, int hidden, int n_ff, int n_expert, int k,
                          float shared_w, void* stream) {
   const char* nm = "sg_moe_layer_noalloc";
-  const size_t need = sg_moe_layer_workspace_bytes(n_tokens, hidden, n_ff, n_expert, k);
+  // (the layout with the shared expert in one group: the layer takes it where
+  // the other one does not fit)
+  const size_t need = n_tokens <= 0 || hidden <= 0 || n_ff <= 0 || n_expert <= 0 || k <= 0
+                          ? 0
+                          : layer_ws(n_tokens, hidden, n_ff, n_expert, k, n_tokens).total;
   if (need > kScratchBytes)
     return set_error(SG_ERR_UNSUPPORTED,
                      "%s: this shape needs %zu B of workspace, more than the %zu B scratch "

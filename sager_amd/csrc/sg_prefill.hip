@@ -21,6 +21,8 @@
 // meet in one lane), K streamed one super-block at a time through two LDS
 // buffers (weights by global_load_lds, token rows gathered through
 // registers).
+#include <cmath>
+
 #include "sg_common.hpp"
 #include "sg_router.hpp"
 
@@ -253,7 +255,7 @@ constexpr int kXRow = 76;
 // run past the tile's rows, into this padding
 constexpr int kXBufWords = (kTokTile * kXRow + 255) / 256 * 256;  // 29 KB
 constexpr int kThreads = 512;                 // eight waves
-constexpr int kDownSlicesPerWg = 8;  // down pass, nb <= 2
+constexpr int kDownSlicesPerWg = 8;  // down pass, nb <= 2, at most
 // LDS: one weight buffer (each wave refills its own rows once it has read
 // them), two token buffers, the tile's token rows and the SiLU's exp table
 // (64 doubles): 78 KB
@@ -778,6 +780,12 @@ __global__ void __launch_bounds__(kPlanThreads) plan_place_kernel(
         off[e1] = ph + h0;
         toff[e1] = pt + t0;
       }
+      // The records' order and sizes set how evenly the grouped kernels'
+      // workgroups end: the shared expert's full tiles first (its rows come
+      // last in the plan), and a group of several tiles cut evenly, in whole
+      // 16-token blocks.
+      const int sh_t = (shared_tail + tok_per - 1) / tok_per;
+      auto even_tile = [](int rows, int n) { return ((rows + n - 1) / n + 15) & ~15; };
       auto put = [&](int t, int g, int p0, int p1, const sg_block_q4k* mg, const sg_block_q4k* mu,
                      const sg_block_q4k* md) {
         const bool present = mg && mu && md;
@@ -793,18 +801,20 @@ __global__ void __launch_bounds__(kPlanThreads) plan_place_kernel(
         if (e >= E) continue;
         if (tiles)
           for (int j = 0; j < tl; ++j) tiles[1 + tb + j] = (e << 16) | j;
-        if (trec)
+        if (trec) {
+          const int per = tl ? even_tile(hq, tl) : 0;
           for (int j = 0; j < tl; ++j)
-            put(tb + j, e, pb + tok_per * j, min(pb + hq, pb + tok_per * (j + 1)), mgp[q], mup[q],
-                mdp[q]);
+            put(sh_t + tb + j, e, pb + min(hq, per * j), pb + min(hq, per * (j + 1)), mgp[q],
+                mup[q], mdp[q]);
+        }
       }
-      const int sh_t = (shared_tail + tok_per - 1) / tok_per;
       if (tiles)
         for (int j = tid; j < sh_t; j += nth) tiles[1 + tot_t + j] = (E << 16) | j;
       if (trec) {
+        const int per = sh_t ? even_tile(shared_tail, sh_t) : 0;
         for (int j = tid; j < sh_t; j += nth)
-          put(tot_t + j, E, tot_h + tok_per * j,
-              min(tot_h + shared_tail, tot_h + tok_per * (j + 1)), sh_g, sh_u, sh_d);
+          put(j, E, tot_h + min(shared_tail, per * j), tot_h + min(shared_tail, per * (j + 1)), sh_g,
+              sh_u, sh_d);
         for (int t = tot_t + sh_t + tid; t < n_rec; t += nth)
           trec[t] = TileRec{-1, 0, 0, 0, 0ull, 0ull, 0ull, 0ull};
       }
@@ -1374,6 +1384,28 @@ size_t sg_moe_prefill_workspace_bytes(int n_tokens, int hidden, int n_ff, int n_
 
 namespace sg {
 
+// The down pass's column slices per workgroup: the rounds that its workgroups
+// take on the chip (two per CU) times the work of one, a slice 1, staging the
+// token rows and the first block 0.6.  Measured per chunk (us, 8 / 4 / 2 / 1
+// slices): 2048 tokens 257 / 258 / 261 / 262 (one full round of 8), with a
+// shared expert 312 / 300 / 299 / 297; 4096 with one 571 / 556 / 566 / 582.
+static int down_slices_per_wg(int n_slices, int T, int k, int E, bool shared) {
+  const double routes = static_cast<double>(T) * k;
+  const double touched = E * (1.0 - std::pow(1.0 - 1.0 / E, routes));  // experts with a route
+  const double tiles = touched * std::ceil(routes / touched / kTokTile) +
+                       (shared ? (T + kTokTile - 1) / kTokTile : 0);
+  int best = 1;
+  double best_cost = 0.0;
+  for (int spw = 1; spw <= kDownSlicesPerWg && n_slices % spw == 0; spw *= 2) {
+    const double cost = std::ceil(tiles * (n_slices / spw) / 512.0) * (spw + 0.6);
+    if (spw == 1 || cost <= best_cost) {
+      best = spw;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
 // the chunk's output: fp32 (residual, out) or the session's fp16 buffers
 struct PrefillOut {
   const float* residual;
@@ -1497,8 +1529,7 @@ static int prefill_launch(const sg_block_q4k* const* tab_gate, const sg_block_q4
   // with at most two super-blocks per row the tile's token rows fit both
   // token buffers, so one workgroup runs several column slices on them
   gd.spw = 1;
-  if (gd.nb <= 2)
-    while (gd.spw < kDownSlicesPerWg && gd.n_slices % (2 * gd.spw) == 0) gd.spw *= 2;
+  if (gd.nb <= 2) gd.spw = down_slices_per_wg(gd.n_slices, n_tokens, k, n_expert, has_shared);
   auto down = [&](auto kern, int n_wg) {
     hipLaunchKernelGGL(kern, dim3(tiles8 * n_wg), dim3(kThreads), kGroupedLds, s, gd);
   };

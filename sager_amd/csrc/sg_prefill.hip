@@ -597,6 +597,9 @@ grouped_mfma_kernel(GroupedArgs a) {
 //    and the tile records.  A row with a duplicated id (caller routing only)
 //    is placed serially in (token, slot) order by workgroup 0 alone, as
 //    dispatch_scan_kernel does.
+// Up to kPlanFusedRows tokens the first launch is left out: every workgroup of
+// the second builds all the bitmaps itself, in LDS, from the ids (a chunk of 57
+// tokens 134.7 -> 130.7 us, of 512 174.5 -> 173.0).
 constexpr int kPlanThreads = 512;
 constexpr int kPlanMaxWg = 256;   // bitmap workgroups; m grows with T beyond 256 * 32 tokens
 
@@ -657,16 +660,19 @@ __global__ void __launch_bounds__(kPlanThreads) plan_bits_kernel(
 // per thread in flight), its own bitmaps (into LDS), its own routes' ids and,
 // in workgroup 0, the experts' matrix pointers.
 constexpr int kColWords = 32;  // bitmap words of one expert's column per thread
+constexpr int kPlanFusedRows = 512;
 
+// kFused: no plan_bits_kernel before it (m = 1; wbits and wflags unused)
+template <bool kFused>
 __global__ void __launch_bounds__(kPlanThreads) plan_place_kernel(
-    const int* __restrict__ idx, const uint32_t* __restrict__ wbits,
+    const int* __restrict__ idx, float* __restrict__ weight, const uint32_t* __restrict__ wbits,
     const int* __restrict__ wflags, int* __restrict__ gslot, int* __restrict__ grows,
     int* __restrict__ off, int* __restrict__ toff, int* __restrict__ meta, int* __restrict__ tiles,
     TileRec* __restrict__ trec, int n_rec, const sg_block_q4k* const* tab_g,
     const sg_block_q4k* const* tab_u, const sg_block_q4k* const* tab_d, const sg_block_q4k* sh_g,
     const sg_block_q4k* sh_u, const sg_block_q4k* sh_d, int n_rows, int k, int E, int m,
     int n_w, int tok_per, int shared_tail) {
-  extern __shared__ __attribute__((aligned(16))) uint32_t pp_lds[];  // own bitmaps [E][m]
+  extern __shared__ __attribute__((aligned(16))) uint32_t pp_lds[];  // own bitmaps [E][m], or all
   __shared__ int hist[1024], pre[1024], offl[1024], part[kPlanThreads];
   __shared__ int s_bad, s_dup, s_tmp[16];
   const int tid = threadIdx.x, nth = blockDim.x, w = blockIdx.x;
@@ -678,7 +684,7 @@ __global__ void __launch_bounds__(kPlanThreads) plan_place_kernel(
   const int wpt = (nwords + tpe - 1) / tpe;
   const int j0 = min(nwords, pq * wpt), j1 = min(nwords, j0 + wpt);
   // --- loads
-  const int f = tid < n_w ? wflags[tid] : 0;  // n_w <= kPlanMaxWg <= nth
+  const int f = !kFused && tid < n_w ? wflags[tid] : 0;  // n_w <= kPlanMaxWg <= nth
   const int ni = (hi - lo) * k;
   int my_e[2];
 #pragma unroll
@@ -687,7 +693,13 @@ __global__ void __launch_bounds__(kPlanThreads) plan_place_kernel(
     const int r = lo + i / k;
     my_e[q] = i < ni ? idx[static_cast<long long>(r) * (k + 1) + (i - (i / k) * k)] : -1;
   }
-  for (int i = tid; i < E * m; i += nth) pp_lds[i] = wbits[static_cast<long long>(w) * E * m + i];
+  // the expert's own-token bitmap word wi (of m) is pp_lds[e * bs + bo + wi]
+  const int bs = kFused ? nwords : m, bo = kFused ? w : 0;
+  if (kFused) {
+    for (int i = tid; i < E * nwords; i += nth) pp_lds[i] = 0u;
+  } else {
+    for (int i = tid; i < E * m; i += nth) pp_lds[i] = wbits[static_cast<long long>(w) * E * m + i];
+  }
   const bool recs = w == 0 && trec;
   const sg_block_q4k* mgp[2] = {nullptr, nullptr};
   const sg_block_q4k* mup[2] = {nullptr, nullptr};
@@ -705,11 +717,35 @@ __global__ void __launch_bounds__(kPlanThreads) plan_place_kernel(
     s_bad = 0;
     s_dup = 0;
   }
+  if (kFused) {  // plan_bits_kernel's work for every token
+    __syncthreads();
+    for (int i = tid; i < n_rows * k; i += nth) {
+      const int r = i / k;
+      const int e = idx[static_cast<long long>(r) * (k + 1) + (i - r * k)];
+      if (e < 0 || e >= E) {
+        if (r >= lo && r < hi) {
+          for (int q = 0; q <= k; ++q) weight[static_cast<long long>(r) * (k + 1) + q] = 0.f;
+          gslot[i] = -1;
+        }
+        atomicAdd(&s_bad, 1);
+        continue;
+      }
+      const uint32_t bit = 1u << (r & 31);
+      if (atomicOr(&pp_lds[e * nwords + (r >> 5)], bit) & bit) s_dup = 1;
+    }
+    __syncthreads();
+  }
   // experts eb + pe, nth / tpe of them per pass (E > nth: one each, several passes)
   for (int eb = 0; eb < E; eb += nth / tpe) {
     const int e = eb + pe;
     int h = 0, p = 0;
-    if (e < E) {
+    if (kFused && e < E) {
+      for (int c = j0; c < j1; ++c) {
+        const int n = __popc(pp_lds[e * nwords + c]);
+        h += n;
+        p += c < w ? n : 0;
+      }
+    } else if (e < E) {
       for (int c0 = j0; c0 < j1; c0 += kColWords) {
         // unconditional loads of clamped addresses (a load under a condition
         // is issued and waited for one at a time), masked afterwards
@@ -852,7 +888,7 @@ __global__ void __launch_bounds__(kPlanThreads) plan_place_kernel(
     const int r = lo + i / k, kk = i - (i / k) * k;
     if (e < 0 || e >= E) return;
     const int d = r - lo, wi = d >> 5;
-    const uint32_t* be = pp_lds + e * m;
+    const uint32_t* be = pp_lds + e * bs + bo;
     int c = offl[e] + pre[e] + __popc(be[wi] & ((1u << (d & 31)) - 1u));
     for (int j = 0; j < wi; ++j) c += __popc(be[j]);
     gslot[r * k + kk] = c;
@@ -1004,16 +1040,41 @@ __global__ void __launch_bounds__(256) prefill_x_kernel(XSrc x, unsigned char* _
   x_block_q8p(x, out, n_blocks, blk, lane);
 }
 
+// sgate[t] = sigmoid(w . x[t]): the shared expert's scalar gate
+// (session.cpp:2904-2909, gemv_f32_out_f16x_batched then
+// sigmoid_gate_scalar_batched_f16), one token per 32-lane half-wave in the
+// reference's fp32 lane order.
+// Workgroup `wg` of 256 threads takes eight tokens.
+__device__ __forceinline__ void shared_gate_wg(const float* __restrict__ w, const XSrc& x,
+                                               float* __restrict__ sgate, int n_tokens, int hidden,
+                                               int wg) {
+  const int l = threadIdx.x & 31;
+  const int t0 = wg * 8 + (threadIdx.x >> 5);
+  const int t = t0 < n_tokens ? t0 : n_tokens - 1;  // whole halves stay active for the shuffles
+  const long long o = static_cast<long long>(t) * hidden;
+  const float g = x.f16 ? rowdot_f32_lanes32(w, [&](int i) { return f16v(x.f16[o + i]); }, hidden, l)
+                        : rowdot_f32_lanes32(w, [&](int i) { return x.f32[o + i]; }, hidden, l);
+  if (l == 0 && t0 < n_tokens) sgate[t0] = sigmoid_sg(g);
+}
+__global__ void __launch_bounds__(256) shared_gate_kernel(const float* __restrict__ w, XSrc x,
+                                                          float* __restrict__ sgate, int n_tokens,
+                                                          int hidden) {
+  shared_gate_wg(w, x, sgate, n_tokens, hidden, blockIdx.x);
+}
+
 // The prefill's first launch: four-wave workgroups.  The first
 // ceil(n_rows / 4) route one token per wave (router_wave, the standalone
 // router's routine); the following ones quantize four blocks of x per wave,
-// so the router's chains and the quantization share one launch.
+// so the router's chains and the quantization share one launch; the last
+// ceil(n_rows / 8) compute the shared expert's gate, when it has one (a launch
+// of its own took 5.3 us).
 constexpr int kRqWaves = 4;
 template <int PL>
 __global__ void __launch_bounds__(64 * kRqWaves) route_quantize_kernel(
     const float* __restrict__ logits, int* __restrict__ idx, float* __restrict__ weight,
     int n_rows, int n_expert, int k, float shared_w, XSrc x, unsigned char* __restrict__ xq,
-    long long n_blocks) {
+    long long n_blocks, int n_qwg, const float* __restrict__ gate_w, float* __restrict__ sgate,
+    int hidden) {
   __shared__ __attribute__((aligned(16))) float ev[kRqWaves][64 * PL];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int n_rwg = (n_rows + kRqWaves - 1) / kRqWaves;  // routing workgroups
@@ -1022,6 +1083,10 @@ __global__ void __launch_bounds__(64 * kRqWaves) route_quantize_kernel(
     if (w < n_rows)
       router_wave<PL>(logits + w * n_expert, n_expert, k, shared_w, idx + w * (k + 1),
                       weight + w * (k + 1), ev[wave], lane);
+    return;
+  }
+  if (static_cast<int>(blockIdx.x) >= n_rwg + n_qwg) {
+    shared_gate_wg(gate_w, x, sgate, n_rows, hidden, blockIdx.x - n_rwg - n_qwg);
     return;
   }
   const long long qw = (static_cast<long long>(blockIdx.x) - n_rwg) * kRqWaves + wave;
@@ -1197,22 +1262,6 @@ __global__ void __launch_bounds__(256) prefill_combine16_kernel(
   *reinterpret_cast<uint4*>(out16 + o) = r;
 }
 
-// sgate[t] = sigmoid(w . x[t]): the shared expert's scalar gate
-// (session.cpp:2904-2909, gemv_f32_out_f16x_batched then
-// sigmoid_gate_scalar_batched_f16), one token per 32-lane half-wave in the
-// reference's fp32 lane order.
-__global__ void __launch_bounds__(256) shared_gate_kernel(const float* __restrict__ w, XSrc x,
-                                                          float* __restrict__ sgate, int n_tokens,
-                                                          int hidden) {
-  const int l = threadIdx.x & 31;
-  const int t0 = blockIdx.x * 8 + (threadIdx.x >> 5);
-  const int t = t0 < n_tokens ? t0 : n_tokens - 1;  // whole halves stay active for the shuffles
-  const long long o = static_cast<long long>(t) * hidden;
-  const float g = x.f16 ? rowdot_f32_lanes32(w, [&](int i) { return f16v(x.f16[o + i]); }, hidden, l)
-                        : rowdot_f32_lanes32(w, [&](int i) { return x.f32[o + i]; }, hidden, l);
-  if (l == 0 && t0 < n_tokens) sgate[t0] = sigmoid_sg(g);
-}
-
 // ---- workspace ------------------------------------------------------------------
 static size_t al256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
@@ -1310,12 +1359,19 @@ static int plan_launch(const int* idx, float* weight, int* gslot, int* grows, in
                      n_rows, E);
   uint32_t* wbits = reinterpret_cast<uint32_t*>(ws + p.wbits);
   int* wflags = reinterpret_cast<int*>(ws + p.wflags);
+  auto place = [&](auto kern, size_t lds) {
+    hipLaunchKernelGGL(kern, dim3(p.n_w), dim3(kPlanThreads), lds, s, idx, weight, wbits, wflags,
+                       gslot, grows, off, toff, meta, tiles, trec, n_rec, pt.g, pt.u, pt.d, pt.sg,
+                       pt.su, pt.sd, n_rows, k, E, p.m, p.n_w, tok_per, shared_tail);
+  };
+  if (n_rows <= kPlanFusedRows) {
+    place(plan_place_kernel<true>, static_cast<size_t>(E) * p.n_w * 4);
+    return check_launch(nm);
+  }
   hipLaunchKernelGGL(plan_bits_kernel, dim3(p.n_w), dim3(kPlanThreads), p.lds_bits, s, idx,
                      weight, gslot, wbits, wflags, n_rows, k, E, p.m);
   if (int st = check_launch(nm)) return st;
-  hipLaunchKernelGGL(plan_place_kernel, dim3(p.n_w), dim3(kPlanThreads), p.lds_bits, s, idx, wbits, wflags,
-                     gslot, grows, off, toff, meta, tiles, trec, n_rec, pt.g, pt.u, pt.d, pt.sg,
-                     pt.su, pt.sd, n_rows, k, E, p.m, p.n_w, tok_per, shared_tail);
+  place(plan_place_kernel<false>, p.lds_bits);
   return check_launch(nm);
 }
 
@@ -1458,11 +1514,12 @@ static int prefill_launch(const sg_block_q4k* const* tab_gate, const sg_block_q4
   if (logits && n_expert <= 512) {  // routing and Q8_K of x in one launch
     const long long nxb = static_cast<long long>(hidden / kQK) * n_tokens;
     const long long qwaves = (nxb + 3) / 4;  // four blocks per wave
-    const unsigned grid = static_cast<unsigned>((n_tokens + kRqWaves - 1) / kRqWaves +
-                                                (qwaves + kRqWaves - 1) / kRqWaves);
+    const int n_qwg = static_cast<int>((qwaves + kRqWaves - 1) / kRqWaves);
+    const unsigned grid = static_cast<unsigned>((n_tokens + kRqWaves - 1) / kRqWaves) + n_qwg +
+                          (sgate ? (n_tokens + 7) / 8 : 0);
     auto launch = [&](auto kern) {
       hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * kRqWaves), 0, s, logits, idx, weight, n_tokens,
-                         n_expert, k, shared_w, x, xq, nxb);
+                         n_expert, k, shared_w, x, xq, nxb, n_qwg, sh_gate_w, sgate, hidden);
     };
     if (n_expert <= 64) launch(route_quantize_kernel<1>);
     else if (n_expert <= 128) launch(route_quantize_kernel<2>);
@@ -1478,11 +1535,11 @@ static int prefill_launch(const sg_block_q4k* const* tab_gate, const sg_block_q4
       if (int st = sg_router_topk(logits, idx, weight, n_expert, k, k + 1, n_tokens, shared_w,
                                   stream))
         return st;
-  }
-  if (sgate) {
-    hipLaunchKernelGGL(shared_gate_kernel, dim3((n_tokens + 7) / 8), dim3(256), 0, s, sh_gate_w, x,
-                       sgate, n_tokens, hidden);
-    if (int st = check_launch("sg_moe_prefill/shared_gate")) return st;
+    if (sgate) {
+      hipLaunchKernelGGL(shared_gate_kernel, dim3((n_tokens + 7) / 8), dim3(256), 0, s, sh_gate_w,
+                         x, sgate, n_tokens, hidden);
+      if (int st = check_launch("sg_moe_prefill/shared_gate")) return st;
+    }
   }
   if (int st = plan_launch(idx, weight, gslot, grows, off, toff, meta, tiles, trec, ws.max_tiles,
                            PlanTables{tab_gate, tab_up, tab_down, sh_gate, sh_up, sh_down},

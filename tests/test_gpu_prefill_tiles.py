@@ -37,3 +37,36 @@ def test_prefill_tiles_bit_exact(H, F, E, k, T, shared):
                                 hidden=H, n_ff=F, k=k, prefill=True)
     np.testing.assert_array_equal(idx.cpu().numpy()[:, :k], ri[:, :k])
     np.testing.assert_array_equal(out.cpu().numpy().view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("n_rows,E,k,dup", [(1, 8, 2, False), (31, 700, 32, False),
+                                            (512, 1024, 32, False), (512, 61, 5, True),
+                                            (513, 61, 5, False), (32, 5, 5, False)])
+def test_plan_of_one_launch(n_rows, E, k, dup):
+    """Up to 512 rows the plan is one launch: every array against the oracle's scan,
+    with invalid ids and (dup) a row that names an expert twice, at its last row
+    count and the two-launch form's first, more and fewer experts than threads,
+    and a full and a partial last group of 32 rows."""
+    rng = np.random.default_rng(n_rows + E)
+    idx = np.stack([rng.choice(E, k, replace=False) for _ in range(n_rows)]).astype(np.int32)
+    idx = np.concatenate([idx, np.full((n_rows, 1), -1, np.int32)], axis=1)
+    if n_rows > 1:
+        idx[n_rows - 1, k - 1] = E
+        idx[n_rows // 2, 0] = -3
+    if dup:
+        idx[n_rows - 3, 1] = idx[n_rows - 3, 0]
+    w = rng.uniform(0, 1, (n_rows, k + 1)).astype(np.float32)
+    ref = orc.dispatch_scan(idx, w, k, E, tok_per=96)
+    wd = torch.from_numpy(w).cuda()
+    got = ops.moe_dispatch_plan(torch.from_numpy(idx).cuda(), wd, E, k, tok_per=96,
+                                shared_tail=n_rows)
+    torch.cuda.synchronize()
+    R = int(ref["meta"][0])
+    host = {n: v.cpu().numpy() for n, v in got.items()}
+    np.testing.assert_array_equal(host["meta"][:3], ref["meta"][:3])
+    np.testing.assert_array_equal(host["off"][:E + 1], ref["off"])
+    np.testing.assert_array_equal(host["toff"][:E + 1], ref["toff"])
+    np.testing.assert_array_equal(host["gslot"], ref["gslot"])
+    np.testing.assert_array_equal(host["grows"][:R], ref["grows"][:R])
+    np.testing.assert_array_equal(host["grows"][R:R + n_rows], np.arange(n_rows))
+    np.testing.assert_array_equal(wd.cpu().numpy(), ref["weight"])

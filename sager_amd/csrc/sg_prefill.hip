@@ -286,6 +286,210 @@ struct GroupedArgs {
                             // to fp16 as the session stores them (session.cpp:2791-2803)
 };
 
+// ---- tiles of a few tokens ---------------------------------------------------------
+// A tile of up to kFewTokens tokens (most experts' while a chunk has fewer routes
+// than a few per expert): the weights are all its work, and what bounds it is how
+// fast they can be unpacked beside the stream.  Its MFMA takes four tokens and
+// four sub-blocks at once instead of sixteen tokens: row 4j + i of A holds token j
+// in K quarter i and zeros in the others, and a lane of K quarter q holds the qs
+// bytes 32q .. 32q + 31 of its weight row, so C element i of a lane is the dot of
+// sub-block 2i (low nibbles) or 2i + 1 (high) of weight row lane & 15 and token
+// lane >> 4.  The nibbles need no scale folded in, the eight scales multiply
+// the lane's eight exact dots, and every lane's outputs are live: per
+// super-block and wave 85 vector instructions, not 175.  The tile's token rows
+// are all staged first, so the waves run free of each other after one
+// barrier, each on its own ring of three weight blocks.
+// Rule: up to 8 tokens, while their rows fit beside the ring.  Per chunk (hidden
+// 2048, n_ff 512, 256 experts, top 8; the general tile / up to 4 tokens / up to 8,
+// us): 33 tokens 99.3 / 83.6 / 84.4, 57 131.2 / 109.6 / 106.3, 130 131.0 / 126.9 /
+// 116.8, 200 145.1 / 142.2 / 132.9, 300 150.2 / 150.3 / 146.5.  At 57 tokens the
+// gate/up launch went from 69 us to 53: 4.7 TB/s of weights.
+constexpr int kFewTokens = 8;
+constexpr int kFewBufs = 3;
+constexpr int kFewXRows = (kWBufWords + 2 * kXBufWords - kFewBufs * kWBufWords) / kXRow - 1;
+constexpr int kFewXInstr = (kFewXRows * 19 + kThreads - 1) / kThreads;
+__device__ __forceinline__ bool few_tokens(int nt, int nb) {
+  return nt <= kFewTokens && nt * nb <= kFewXRows;
+}
+
+// ma: the wave's matrix; slices: column slices from c0 on, in turn
+template <bool kGateUp, bool kF16Out>
+__device__ __forceinline__ void few_tile(const GroupedArgs& a, const sg_block_q4k* mw,
+                                         uint32_t* lds, double* etab, int p0, int nt, int c0,
+                                         int slices) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lr = lane & 15, lq = lane >> 4;
+  const int nb = a.nb, n = slices * nb;
+  constexpr int kCols = kGateUp ? kRowsWg / 2 : kRowsWg;
+  constexpr int kWChunks = kRowsWg * 9 / 8;
+  const int ng = (nt + 3) >> 2;
+  // token rows by scalar loads (the constant address space): a vector load's wait
+  // would wait for the weight copies before it too
+  const int __attribute__((address_space(4)))* grows =
+      (const int __attribute__((address_space(4)))*)(reinterpret_cast<uintptr_t>(uniform_ptr(a.grows)));
+  const int pu = __builtin_amdgcn_readfirstlane(p0), nu = __builtin_amdgcn_readfirstlane(nt);
+  int rows[kFewTokens];
+#pragma unroll
+  for (int t = 0; t < kFewTokens; ++t) rows[t] = kGateUp ? grows[pu + min(t, nu - 1)] : pu + t;
+  const double ev = kGateUp ? kExp2Tab64[lane] : 0.0;
+  uint32_t* ring = lds + 4 * wave * kWChunks;
+  uint32_t* x = lds + kFewBufs * kWBufWords;
+  uint32_t* zero = x + nt * nb * kXRow;
+  // chunk c of the wave's 16 rows: part c % 9 of row c / 9; step i (slice i / nb,
+  // block i % nb) goes in the scalar offset
+  const u32x4 rw4 = buffer_desc(mw, a.n_rows * nb * kQ4Bytes);
+  uint32_t wofs[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int cc = min(wave * kWChunks + lane + 64 * i, kRowsWg * 9 - 1);
+    const int row = cc / 9, part = cc - row * 9;
+    wofs[i] = static_cast<uint32_t>((c0 + (kGateUp ? (row & 63) : row)) * nb) * kQ4Bytes + 16 * part;
+  }
+  int is_b = 0;
+  uint32_t is_ofs = 0;  // the next step to copy
+  auto stage = [&](int slot) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      if (64 * i + lane < kWChunks)
+        dma16(ring + slot * kWBufWords + 256 * i, wofs[i], rw4, is_ofs + is_b * kQ4Bytes);
+    if (++is_b == nb) {
+      is_b = 0;
+      is_ofs += static_cast<uint32_t>(kCols * nb) * kQ4Bytes;
+    }
+  };
+  stage(0);
+  // the token rows, whole: token t's blocks at x + t nb kXRow
+  {
+    const u32x4 rx4 = buffer_desc(a.xq, 0x7FFFFFFFu);
+    const int per = nb * 19, total = nt * per;
+#pragma unroll
+    for (int i = 0; i < kFewXInstr; ++i) {
+      const int cb = kThreads * i + 64 * wave, c = cb + lane;
+      if (cb >= total) break;
+      int row = rows[0], at = c;
+#pragma unroll
+      for (int u = 1; u < kFewTokens; ++u)
+        if (c >= u * per) {
+          row = rows[u];
+          at = c - u * per;
+        }
+      if (c < total)
+        dma16(x + 4 * cb, static_cast<uint32_t>(row * nb) * kQ8PBytes + 16 * at, rx4, 0);
+    }
+  }
+  if (tid < kXRow) zero[tid] = 0;
+#pragma unroll
+  for (int i = 1; i < kFewBufs; ++i)
+    if (i < n) stage(i);
+  wait_vm_sets<kFewBufs - 1, 3>(min(kFewBufs - 1, n - 1));  // the first block and the token rows
+  bar();
+  // A row lr: token lr >> 2 (of its group of four), the lane's quarter if (lr & 3) == lq;
+  // the mins' row 4j: token j; tokens past nt and the other quarters read zeros
+  const uint32_t *xa0[2], *xm0[2], *xd0[2];
+  int sa[2], sm_[2], sd[2];
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    const int tr = 4 * g + (lr >> 2), tq = 4 * g + lq;
+    const bool va = tr < nt && (lr & 3) == lq, vm = tr < nt, vd = tq < nt;
+    xa0[g] = (va ? x + tr * nb * kXRow : zero) + 4 + 16 * lq;
+    xm0[g] = (vm ? x + tr * nb * kXRow : zero) + 68 + 2 * lq;
+    xd0[g] = vd ? x + tq * nb * kXRow : zero;
+    sa[g] = va ? kXRow : 0;
+    sm_[g] = vm ? kXRow : 0;
+    sd[g] = vd ? kXRow : 0;
+  }
+  float acc[2] = {0.f, 0.f};
+  int slot = 0, b = 0;
+#pragma unroll 1
+  for (int i = 0; i < n; ++i) {
+    wait_vm_sets<kFewBufs - 1, 3>(min(kFewBufs - 1, n - 1 - i));
+    const uint32_t* Wl = ring + slot * kWBufWords + lr * kWRowWords;
+    const uint4 whdr = *reinterpret_cast<const uint4*>(Wl);
+    const uint4 q0 = *reinterpret_cast<const uint4*>(Wl + 4 + 8 * lq);
+    const uint4 q1 = *reinterpret_cast<const uint4*>(Wl + 8 + 8 * lq);
+    wait_lds();
+    if (i + kFewBufs < n) stage(slot);
+    slot = slot == kFewBufs - 1 ? 0 : slot + 1;
+    const ScaleMins sm = unpack_scales(whdr.y, whdr.z, whdr.w);
+    auto lo = [](uint32_t v) { return static_cast<int>(v & 0x0F0F0F0Fu); };
+    auto hi = [](uint32_t v) { return static_cast<int>((v >> 4) & 0x0F0F0F0Fu); };
+    const v4i l0 = {lo(q0.x), lo(q0.y), lo(q0.z), lo(q0.w)};
+    const v4i l1 = {lo(q1.x), lo(q1.y), lo(q1.z), lo(q1.w)};
+    const v4i h0 = {hi(q0.x), hi(q0.y), hi(q0.z), hi(q0.w)};
+    const v4i h1 = {hi(q1.x), hi(q1.y), hi(q1.z), hi(q1.w)};
+    v4h bmn;  // the mins term of the general tile
+    {
+      const uint32_t mw2 = (lq & 1) ? sm.mn_hi : sm.mn_lo;
+      const uint32_t m2 = lq < 2 ? mw2 << 1 : mw2;
+      const h2 k1024 = {static_cast<_Float16>(-1024.f), static_cast<_Float16>(-1024.f)};
+      const h2 f0 = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, m2, 0x04010400u)) + k1024;
+      const h2 f1 = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, m2, 0x04030402u)) + k1024;
+      bmn = v4h{f0.x, f0.y, f1.x, f1.y};
+    }
+    const float d = half_bits_to_float(whdr.x & 0xFFFFu);
+    const float dmin = half_bits_to_float(whdr.x >> 16);
+    auto sc = [&](int sb) {
+      return static_cast<int>(((sb < 4 ? sm.sc_lo : sm.sc_hi) >> (8 * (sb & 3))) & 0xFFu);
+    };
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      if (g >= ng) continue;
+      const v4i* xp = reinterpret_cast<const v4i*>(xa0[g] + b * sa[g]);
+      const v4h ab = *reinterpret_cast<const v4h*>(xm0[g] + b * sm_[g]);
+      const float xd = __builtin_bit_cast(float, xd0[g][b * sd[g]]);
+      v4i cl = {0, 0, 0, 0}, ch = cl;
+      cl = __builtin_amdgcn_mfma_i32_16x16x64_i8(xp[0], l0, cl, 0, 0, 0);
+      ch = __builtin_amdgcn_mfma_i32_16x16x64_i8(xp[2], h0, ch, 0, 0, 0);
+      cl = __builtin_amdgcn_mfma_i32_16x16x64_i8(xp[1], l1, cl, 0, 0, 0);
+      ch = __builtin_amdgcn_mfma_i32_16x16x64_i8(xp[3], h1, ch, 0, 0, 0);
+      const v4f mf = __builtin_amdgcn_mfma_f32_16x16x16f16(ab, bmn, v4f{}, 0, 0, 0);
+      int I = 0;  // |dot| <= 32 * 15 * 127: 24 bits
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        I += __mul24(sc(2 * u), cl[u]) + __mul24(sc(2 * u + 1), ch[u]);
+      const float t = __builtin_fmaf(d, static_cast<float>(I), -(dmin * mf[0]));
+      acc[g] = __builtin_fmaf(xd, t, acc[g]);
+    }
+    if (++b < nb) continue;
+    b = 0;
+    if constexpr (!kGateUp) {  // a slice's outputs
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const int tt = 4 * g + lq;
+        if (tt < nt) {
+          const long long o = static_cast<long long>(p0 + tt) * a.n_out + c0 + 16 * wave + lr;
+          if (kF16Out) a.out16[o] = f16b(acc[g]);
+          else a.out[o] = acc[g];
+        }
+        acc[g] = 0.f;
+      }
+      c0 += kCols;
+    }
+  }
+  if constexpr (kGateUp) {
+    // h = silu(gate) * up: gate wave w takes tokens 0-3, up wave w + 4 tokens 4-7,
+    // each getting the other's half through that wave's first ring slot (its
+    // copies have all landed and been read)
+    const bool up_wave = wave >= 4;
+    ring[lane] = __builtin_bit_cast(uint32_t, up_wave ? acc[0] : acc[1]);
+    if (wave == 7) etab[lane] = ev;
+    bar();
+    const float other = __builtin_bit_cast(float, lds[4 * (wave ^ 4) * kWChunks + lane]);
+    const int tt = 4 * up_wave + lq;
+    float gv[1] = {up_wave ? other : acc[0]}, uv[1] = {up_wave ? acc[1] : other}, hv[1];
+    if (a.r16) {
+      gv[0] = f16r(gv[0]);
+      uv[0] = f16r(uv[0]);
+    }
+    if (tt < nt) {
+      silu_mul_tab_n<1>(gv, uv, hv, etab);
+      const long long o = static_cast<long long>(p0 + tt) * a.n_out + c0 + 16 * (wave & 3) + lr;
+      if (a.r16) a.out16[o] = f16b(f16r(hv[0]));
+      else a.out[o] = hv[0];
+    }
+  }
+}
+
 // One workgroup = one column slice of one tile (up to 128 positions of one
 // group).  The 1-D grid is laid out so that every slice of a tile runs on
 // one XCD and is dispatched together: workgroup L runs on XCD L % 8, and
@@ -340,6 +544,10 @@ grouped_mfma_kernel(GroupedArgs a) {
   // in the scalar offset (buffer_load ... lds).
   constexpr int kWChunks = kRowsWg * 9 / 8;  // 144 per wave
   const sg_block_q4k* mw = uniform_ptr((kGateUp && wave >= 4) ? mb : ma);
+  if (few_tokens(p1 - p0, nb)) {
+    few_tile<kGateUp, kF16Out>(a, mw, gl_lds, etab, p0, p1 - p0, c0, spw);
+    return;
+  }
   const u32x4 rw4 = buffer_desc(mw, a.n_rows * nb * kQ4Bytes);
   uint32_t wofs[3];
   auto set_wofs = [&](int cs) {  // the per-lane chunk offsets of slice columns cs ..
@@ -1450,9 +1658,13 @@ static int down_slices_per_wg(int n_slices, int T, int k, int E, bool shared) {
   const double touched = E * (1.0 - std::pow(1.0 - 1.0 / E, routes));  // experts with a route
   const double tiles = touched * std::ceil(routes / touched / kTokTile) +
                        (shared ? (T + kTokTile - 1) / kTokTile : 0);
+  // Tiles of a few tokens stage little, and short workgroups fill in beside the
+  // longer tiles: 57 tokens 106.8 with 2 slices, 107.6 / 120.1 with 4 / 8; 130
+  // tokens 117.2, 117.9 / 119.7; 20, 33 and 200 alike with 2 to 8.
+  const int most = routes <= kFewTokens * touched ? 2 : kDownSlicesPerWg;
   int best = 1;
   double best_cost = 0.0;
-  for (int spw = 1; spw <= kDownSlicesPerWg && n_slices % spw == 0; spw *= 2) {
+  for (int spw = 1; spw <= most && n_slices % spw == 0; spw *= 2) {
     const double cost = std::ceil(tiles * (n_slices / spw) / 512.0) * (spw + 0.6);
     if (spw == 1 || cost <= best_cost) {
       best = spw;

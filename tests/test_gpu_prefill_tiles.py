@@ -70,3 +70,33 @@ def test_plan_of_one_launch(n_rows, E, k, dup):
     np.testing.assert_array_equal(host["grows"][:R], ref["grows"][:R])
     np.testing.assert_array_equal(host["grows"][R:R + n_rows], np.arange(n_rows))
     np.testing.assert_array_equal(wd.cpu().numpy(), ref["weight"])
+
+
+# (hidden, n_ff, tokens): every token of the one expert in one tile.  One weight
+# block, one slice; one, four, five and eight tokens; the first tile past them; 73 and
+# 74 staged blocks (the most, and one too many: the general tile); three blocks per
+# down row, where its workgroups take one slice
+FEW = [(256, 256, 1), (512, 256, 4), (512, 512, 5), (2048, 512, 8), (2048, 512, 9),
+       (73 * 256, 256, 1), (37 * 256, 256, 2), (256, 37 * 256, 2), (512, 768, 3)]
+
+
+@pytest.mark.parametrize("H,F,T", FEW)
+@pytest.mark.parametrize("f16", [False, True])
+def test_few_token_tiles_bit_exact(H, F, T, f16):
+    rng = np.random.default_rng(H + F + T)
+    mats = [q4k_random_np(rng, F * H // 256) for _ in range(3)]
+    dev = [torch.from_numpy(m).cuda() for m in mats]
+    tabs = [torch.tensor([m.data_ptr()], dtype=torch.int64, device="cuda") for m in dev]
+    pre = ops.MoePrefill(*tabs, None, hidden=H, n_ff=F, n_expert=1, k=1, max_tokens=T)
+    x = rng.normal(0, 1, (T, H)).astype(np.float16 if f16 else np.float32)
+    lg = rng.normal(0, 1, (T, 1)).astype(np.float32)
+    args = ([mats[0]], [mats[1]], [mats[2]], None, x)
+    kw = dict(logits=lg, hidden=H, n_ff=F, k=1, prefill=True)
+    if f16:
+        out, _, _ = pre.forward_f16(torch.from_numpy(x).cuda(), None, torch.from_numpy(lg).cuda())
+        ref = orc.moe_layer_f16(*args, **kw)[0]
+    else:
+        out, _, _ = pre.forward(torch.from_numpy(x).cuda(), torch.from_numpy(lg).cuda())
+        ref = orc.moe_layer(*args, **kw)[0]
+    bits = np.uint16 if f16 else np.uint32
+    np.testing.assert_array_equal(out.cpu().numpy().view(bits), ref.view(bits))

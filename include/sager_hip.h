@@ -256,7 +256,7 @@ int sg_gemv_f32_out_f16x(const float* w, const uint16_t* x, float* y, int n_rows
  *   out:      fp32 [n_tokens][hidden].
  *   idx, weight: [n_tokens][k+1] (slot k of weight = shared_w).
  *   workspace: device buffer of at least sg_moe_layer_workspace_bytes()
- *             (scratch: the plan and h between the two launches).
+ *             (scratch: the plan and h between the launches).
  * The reference applies the gate to the shared output before the combine,
  * so slot k adds fma(shared_w, y_shared * sigmoid(g), acc); weight[t][k]
  * stays shared_w.
@@ -328,9 +328,10 @@ int sg_moe_layer_noalloc(const sg_block_q4k* const* tab_gate,
                          float* out, int* idx, float* weight, int n_tokens, int hidden,
                          int n_ff, int n_expert, int k, float shared_w, void* stream);
 
-/* The two launches of sg_moe_layer, selectable: bit 0 = front (top-k,
- * Q8_K of x, the expert-major plan, gate/up GEMV + SiLU), bit 1 = back
- * (Q8_K of h, down GEMV, combine).  The back stage reads what the front left
+/* The two stages of sg_moe_layer, selectable: bit 0 = front (top-k,
+ * Q8_K of x, the expert-major plan, gate/up GEMV + SiLU and, for several
+ * tokens, Q8_K of h), bit 1 = back (Q8_K of h if it is still to do, down
+ * GEMV, combine).  The back stage reads what the front left
  * in `workspace`, so a caller may run them separately on one stream (to put
  * other work between them, or to time one); stages = 3 is sg_moe_layer.
  * The reference issues these steps as separate launchers from
@@ -366,8 +367,8 @@ int sg_moe_dispatch_scan(const int* idx, float* weight, int* gslot, int* grows,
                          int* off, int* toff, int* meta, int n_rows, int k,
                          int n_expert, int tok_per, void* stream);
 
-/* The same plan built by two launches over many workgroups (32 tokens
- * each: bitmaps, then offsets and placement), with no
+/* The same plan built over many workgroups (32 tokens each: bitmaps, then
+ * offsets and placement; one launch up to 512 rows, else two), with no
  * limit on n_rows beyond int indexing; the order inside an expert is the
  * same (token, then slot), so every array equals sg_moe_dispatch_scan's.
  * It is the plan sg_moe_prefill builds.  Extra outputs:

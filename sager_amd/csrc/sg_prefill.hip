@@ -15,7 +15,7 @@
 // the super-blocks in order (the integer-first order; the CPU oracle's
 // orc_gemv_q4k_q8_int is the same arithmetic).
 //
-// Workgroup tile: 64 tokens x 128 weight rows (gate/up: 64 h rows of gate
+// Workgroup tile: up to 96 tokens x 128 weight rows (gate/up: 64 h rows of gate
 // and the same 64 of up; down: 128 output rows), eight waves of 16 tokens x
 // 64 rows each (gate/up: 32 h rows of gate and their up rows, so SiLU pairs
 // meet in one lane), K streamed one super-block at a time through two LDS

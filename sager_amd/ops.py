@@ -278,7 +278,7 @@ class MoeLayer:
     """One MoE layer's device-side pointer tables and workspace; ``forward``
     is the device-path dispatch of Session::moe_dispatch_device
     (session.cpp:2482-3030) as one call.  ``stages``: 3 = front and back (the
-    whole layer), 1 / 2 = one of the two launches.  ``shared_gate_w``: the
+    whole layer), 1 / 2 = one of the two stages.  ``shared_gate_w``: the
     shared expert's fp32 [hidden] gate row (LayerWeights::shared_gate_w), or
     None."""
 

@@ -1541,13 +1541,19 @@ layer_gateup_kernel(LayerArgs args) {
     dma_gateup(reinterpret_cast<const sg_block_q4k*>(wg), reinterpret_cast<const sg_block_q4k*>(wu),
                row0, nrw, nbh, wbuf[wave], lane);
   // the first entry's x (quantized by the routing launch) beside the
-  // weights, one copy instruction per wave
+  // weights, its 1-KB copy instructions (up to ten) dealt to the waves
   uint32_t* x0 = dyn;
   if (n > 0) {
     const int t0 = ent1 ? __shfl(v_tok, j0, 64) : a.plan.tok[j0];
     const uint32_t* src = a.xq + static_cast<long long>(t0) * xw;
-    dma_chunks([&](int c) { return reinterpret_cast<const char*>(src) + 16 * c; }, xw / 4, x0,
-               lane, wave, 4);
+    dma_chunks([&](int c) { return reinterpret_cast<const char*>(src) + 16 * c; },
+               min(xw / 4, 576), x0, lane, wave, 4);
+    // past hidden 7168 x is more than the 576 chunks of nine instructions: a
+    // tenth, wave 1's turn (hidden <= 8192: 640 chunks).  One loop over all
+    // chunks instead made the batch of 13 tokens 3 % slower.
+    if (NBH == 0 && wave == 1 && 576 + lane < xw / 4)
+      __builtin_amdgcn_global_load_lds((glb_void_p)(src + 4 * (576 + lane)),
+                                       (lds_void_p)(x0 + 4 * 576), 16, 0, 0);
   }
   int* etok = reinterpret_cast<int*>(dyn + ((xw + 3) & ~3));
   int* eslot = etok + a.emax;

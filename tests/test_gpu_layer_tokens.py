@@ -14,11 +14,14 @@ pytestmark = pytest.mark.gpu
 # no power of two; an odd expert table; more than 64, 128, 256 and 512 experts (the
 # routing instances); 47 and 48 h blocks (quantized by the back kernel, by a launch
 # of its own); groups of the shared expert full and not; the most slots that
-# LDS holds
+# LDS holds; the first entry's x in 560, 580 and (the widest hidden) 640 16-B chunks,
+# where a wave's nine copy instructions hold 576
 CASES = [(256, 256, 8, 1, 2, False), (512, 256, 61, 7, 16, True), (1280, 768, 60, 7, 5, True),
          (768, 256, 130, 8, 13, True), (256, 256, 300, 23, 2, False),
          (256, 256, 70, 22, 2, True),
-         (256, 256, 600, 11, 4, False), (512, 512, 32, 5, 4, True), (512, 256, 33, 32, 11, True)]
+         (256, 256, 600, 11, 4, False), (512, 512, 32, 5, 4, True), (512, 256, 33, 32, 11, True),
+         (7168, 256, 5, 2, 2, True), (7424, 256, 5, 2, 3, False), (8192, 256, 6, 3, 2, False),
+         (8192, 256, 9, 2, 10, True)]
 
 
 def _layer(rng, H, F, E, k, T, shared):

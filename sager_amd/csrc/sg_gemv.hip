@@ -312,10 +312,9 @@ __global__ void __launch_bounds__(64 * kLatWaves) gemv_lat_plain_kernel(
   gemv_lat_body(PlainRows{w, nb}, xq, F32Out{y}, n_rows, nb, lg);
 }
 
-// y[t*n_rows + r] = W[r] . x[t] for the few tokens of short rows
-// (n_tokens * nb <= 8) in large matrices: a lane per super-block as in
-// gemv1_kernel, looping over the tokens with sdot4.  The matrix-core kernels
-// below win everywhere else.
+// y[t*n_rows + r] = W[r] . x[t] for two to four tokens of large matrices: a
+// lane per super-block as in gemv1_kernel, looping over the tokens with sdot4.
+// The matrix-core kernels below win outside use_batched_sdot's ranges.
 template <typename Out>
 __global__ void __launch_bounds__(256) gemv_batched_kernel(const sg_block_q4k* __restrict__ w,
                                                            const unsigned char* __restrict__ xq,
@@ -814,20 +813,41 @@ static int launch_ptrs(const sg_block_q4k* const* ptrs, const sg_block_q8k* x, O
 }
 
 // Which several-token kernel, by super-blocks (n_rows * nb), measured cold in
-// graphs (us, quantizer included):
-// - gemv_batched_kernel: at most eight staged blocks of two to four tokens in
-//   a matrix of 65536 or more (262141 x 512: 2 tokens 17.8 against 20.4 for
-//   the streaming kernel; 3 tokens 19.7 / 20.6; 4 tokens x 1024 23.1 / 20.3);
-// - gemv_mtw_kernel, the streaming one: from 131072 with more than 8 blocks
-//   per row (8197 x 4096: 11.5 against 13.7; 4096 x 4096: 8.3 / 7.4), from
-//   262144 below that (32765 x 2048: 12.9 / 15.2; 16381 x 2048: 10.0 / 10.0); with
-//   more than 8 tokens, whose sets are twice the work, from 524288 (65533 x
-//   2048: 23.7 / 26.0; 32765: 15.8 / 15.7) and only with more than 4 blocks
-//   per row (131069 x 1024: 25.8 / 22.6);
+// graphs (us; sdot4 / matrix cores):
+// - gemv_batched_kernel, the sdot4 one:
+//   - at most eight staged blocks of two to four tokens from 65536 blocks on
+//     (262141 x 512, 2 tokens 17.8 / 20.4, 3 tokens 19.7 / 20.6; 4 tokens x
+//     1024 23.1 / 20.3);
+//   - two tokens of 6 to 8 blocks per row from 150000 on (18750 x 2048 9.7 /
+//     10.0, 37449 x 1792 12.4 / 14.6, 52500 x 2048 17.0 / 17.0, 250000 x 2048
+//     56.6 / 59.0, but 14285 x 1792 7.9 / 7.3), of 5 up to the streaming kernel's
+//     line (46000 x 1280 12.5 / 13.3, 60000 x 1280 15.3 / 13.4);
+//   - two or three tokens of 17 to 32 blocks per row, which the streaming
+//     kernel does not take and for which gemv_mt_kernel needs two chunks, in
+//     rounds of 4096 rows (16 per CU).  Two tokens: past three rounds (12400 x
+//     5120 18.3 / 21.5, 152064 x 5120 138 / 190) and while the third is less than
+//     half full (9000 x 6144 17.0 / 18.3, 11000 x 6144 19.5 / 19.1, 8192 x 8192
+//     19.3 / 16.9); past 32 blocks half of its lanes idle (60606 x 8448 134 /
+//     114).  Three tokens: from 786432 blocks up to 20 per row (58823 x 4352 70.1 /
+//     75.8, 35000 x 5120 50.9 / 49.6), from 700000 at 32, where every lane has a
+//     block (21875 x 8192 44.8 / 48.0, 18750 x 8192 42.4 / 40.4), from 1048576
+//     between (41666 x 7680 73.7 / 77.5, 25000 x 7168 46.4 / 45.8, 36363 x 5632
+//     54.6 / 51.4).  Four tokens: never (152064 x 5120 223 / 200);
+// - gemv_mtw_kernel, the streaming one (us; gemv_mt_kernel / this one): from
+//   131072 with more than 8 blocks per row (8197 x 4096 13.7 / 11.5; 4096 x 4096
+//   7.4 / 8.3), from 262144 below that (32765 x 2048 15.2 / 12.9; 16381 x 2048
+//   10.0 / 10.0); with more than 8 tokens, whose sets are twice the work, from
+//   524288 (65533 x 2048 26.0 / 23.7; 32765 15.7 / 15.8) and only with more than
+//   4 blocks per row (131069 x 1024 22.6 / 25.8);
 // - gemv_mt_kernel otherwise.
 static bool use_batched_sdot(int n_rows, int nb, int n_tokens) {
-  return n_tokens >= 2 && n_tokens <= 4 && n_tokens * nb <= 8 &&
-         static_cast<long long>(n_rows) * nb >= 65536;
+  const long long blocks = static_cast<long long>(n_rows) * nb;
+  if (n_tokens < 2 || n_tokens > 4) return false;
+  if (n_tokens * nb <= 8) return blocks >= 65536;
+  if (n_tokens == 2 && nb <= 8) return blocks >= 150000 && (nb > 5 || blocks < 262144);
+  if (nb <= 16 || nb > 32) return false;
+  if (n_tokens == 2) return n_rows > 12288 || (n_rows > 8192 && n_rows <= 10240);
+  return n_tokens == 3 && blocks >= (nb <= 20 ? 786432 : nb < 32 ? 1048576 : 700000);
 }
 static bool use_mtw(int n_rows, int nb, int n_tokens) {
   if (nb < 2 || nb > 16 || (n_tokens > 8 && nb <= 4)) return false;

@@ -14,14 +14,19 @@ pytestmark = pytest.mark.gpu
 
 # rows: below, at and past a 16-row set.  Below 131072 (more than 8 blocks per
 # row), 262144 or (more than 8 tokens) 524288 super-blocks the direct kernel,
-# from there on the streaming one, with ragged last sets; few tokens of short
-# rows the sdot4 kernel; one token the one-token GEMV.  k: one block, counts that
-# are no power of two, the streaming kernel's last (16), chunks of 16 blocks with
-# a ragged last one.  Tokens: the token tiles of 8 and 16, full and not.
+# from there on the streaming one, with ragged last sets; one token the one-token
+# GEMV.  k: one block, counts that are no power of two, the streaming kernel's last
+# (16), chunks of 16 blocks with a ragged last one.  Tokens: the token tiles of 8
+# and 16, full and not.  The last three lines: both sides of the sdot4 kernel's
+# lines (two to four tokens of short rows, two of 5 to 8 blocks, two and three of
+# 17 to 32).
 CASES = [(1, 256, 1), (15, 2048, 2), (17, 1280, 3), (16, 768, 7), (64, 4096, 16), (33, 4352, 5),
          (16000, 4352, 3), (70001, 256, 4), (65539, 256, 16), (131077, 512, 5),
          (87395, 768, 8), (37450, 1792, 4), (32769, 2048, 3), (65537, 2048, 16),
-         (104861, 1280, 9), (14564, 2304, 5), (8193, 4096, 2), (8200, 4096, 16)]
+         (104861, 1280, 9), (14564, 2304, 5), (8193, 4096, 2), (8200, 4096, 16),
+         (16381, 1024, 2), (65537, 256, 2), (29999, 1280, 2), (30001, 1280, 2), (52429, 1280, 2),
+         (25001, 1536, 2), (18751, 2048, 2), (32771, 2048, 2), (8192, 4352, 2), (8193, 5632, 2),
+         (10241, 4352, 2), (12289, 8192, 2), (12289, 8448, 2), (46261, 4352, 3), (21876, 8192, 3)]
 
 
 @pytest.mark.parametrize("n_rows,k,T", CASES)

@@ -1733,9 +1733,11 @@ __device__ __forceinline__ void back_combine(const LayerArgs& a, const BackLds& 
 // time (0 = read from a).  pre: the kernel start has already issued every
 // group's down-row copies (the packed one-pass layout) and quantized h,
 // and the barrier after them has passed.
-// kAhead: a pass's rows are issued during the pass before.  The one-token shape's
-// instances have one pass and go without: with the copies out of line for a
-// second pass that never comes, the kernel took 5.42 us instead of 4.94.
+// kAhead: a pass's rows are issued during the pass before.  The one-token model
+// shape's instances have one pass and go without: with the copies out of line for
+// a second pass that never comes, the kernel took 5.42 us instead of 4.94.  Other
+// one-token shapes run faster with them, also in one pass (hidden 1280, n_ff 768
+// 14.7 us against 15.3; 1024, 512 7.6 / 8.0; 2048, 512 7.37 / 7.34).
 template <int NBF, int ROWS, int HS, bool kAhead>
 __device__ __forceinline__ void back_core(const LayerArgs& a, const BackLds& L, uint32_t* bd,
                           uint32_t (*wbuf)[64 * 36], int row0, int nr, float res0,
@@ -1971,12 +1973,20 @@ __device__ __forceinline__ float residual_pre(const LayerArgs& a, int row0, int 
   return a.residual ? a.residual[o] : f16v(a.res16[o]);
 }
 
-template <int NBF, int ROWS, int kShapeT = 0, bool kSh = false, int kIo = 0>
+// kOne: one token, whose h is never quantized before this launch: constants, also
+// where the shape is not.  The back stage of hidden 2048, n_ff 512 without / with
+// (us): 128 experts, top 8 7.71 / 7.37; 512, top 10 9.05 / 8.70; 128, top 16
+// 11.6 / 11.2; 64, top 6 7.19 / 6.87.
+template <int NBF, int ROWS, int kShapeT = 0, bool kSh = false, int kIo = 0, bool kOne = kShapeT == 1>
 __global__ void __launch_bounds__(kBackThreads) layer_back_kernel(LayerArgs args) {
   // kShapeT > 0 (the model shape with kShapeT tokens, as in the front
   // kernel): the shape and the LDS layout are constants
   LayerArgs a = args;
   apply_shape<kShapeT, kSh, kIo>(a);
+  if constexpr (kOne) {
+    a.T = 1;
+    a.hq_pre = 0;
+  }
   if constexpr (kShapeT > 0) {
     a.back_rows = 8;
     a.back_lrow = 2;
@@ -2436,6 +2446,12 @@ static int layer_launch(const sg_block_q4k* const* tab_gate, const sg_block_q4k*
         hipLaunchKernelGGL((layer_back_kernel<2, 8, kShapeWindow, true, 2>), gb, dim3(kBackThreads),
                            lds_bb, s, a);
     }
+    else if (one && n_ff / kQK == 2 && rows == 8)
+      hipLaunchKernelGGL((layer_back_kernel<2, 8, 0, false, 0, true>), gb, dim3(kBackThreads),
+                         lds_b + back_bufs * buf_b, s, a);
+    else if (one)
+      hipLaunchKernelGGL((layer_back_kernel<0, 0, 0, false, 0, true>), gb, dim3(kBackThreads),
+                         lds_b + back_bufs * buf_b, s, a);
     else if (n_ff / kQK == 2 && rows == 8)
       hipLaunchKernelGGL((layer_back_kernel<2, 8>), gb, dim3(kBackThreads),
                          lds_b + back_bufs * buf_b, s, a);

@@ -15,13 +15,15 @@ pytestmark = pytest.mark.gpu
 # routing instances); 47 and 48 h blocks (quantized by the back kernel, by a launch
 # of its own); groups of the shared expert full and not; the most slots that
 # LDS holds; the first entry's x in 560, 580 and (the widest hidden) 640 16-B chunks,
-# where a wave's nine copy instructions hold 576
+# where a wave's nine copy instructions hold 576; one token of other shapes than the
+# model's (its down copies at the kernel's start and, with more groups, later)
 CASES = [(256, 256, 8, 1, 2, False), (512, 256, 61, 7, 16, True), (1280, 768, 60, 7, 5, True),
          (768, 256, 130, 8, 13, True), (256, 256, 300, 23, 2, False),
          (256, 256, 70, 22, 2, True),
          (256, 256, 600, 11, 4, False), (512, 512, 32, 5, 4, True), (512, 256, 33, 32, 11, True),
          (7168, 256, 5, 2, 2, True), (7424, 256, 5, 2, 3, False), (8192, 256, 6, 3, 2, False),
-         (8192, 256, 9, 2, 10, True)]
+         (8192, 256, 9, 2, 10, True), (2048, 512, 20, 16, 1, True), (512, 768, 12, 7, 1, True),
+         (2048, 512, 70, 10, 1, False), (8192, 256, 5, 3, 1, True)]
 
 
 def _layer(rng, H, F, E, k, T, shared):

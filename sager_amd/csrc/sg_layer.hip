@@ -974,8 +974,8 @@ __device__ __forceinline__ void shared_gate_tokens(const LayerArgs& a, int tid, 
 // routing (streaming the exact expert instead when they differ) and writes
 // h for the entry of its group in the exact plan.  The publisher workgroup
 // (g == gmax, bx == 0) runs the same routing and writes idx, weight and the
-// plan; the next one of its row (bx == 1), otherwise idle, computes the shared
-// expert's gate.
+// plan; the next one of its row (bx == 1; n_ff >= 256 makes two chunks or more),
+// otherwise idle, computes the shared expert's gate.
 // NBH: hidden / 256 when compiled for it (0 = read from a).
 template <int EPT, int NBH>
 __device__ __forceinline__ void front_body(const LayerArgs& a, int bx, int g, uint32_t (*wbuf)[64 * 36],
@@ -1040,8 +1040,6 @@ __device__ __forceinline__ void front_body(const LayerArgs& a, int bx, int g, ui
     gateup_wave(true, row0, nrw, nbh, lpr, buf, xs,
                 [&](int, int& t, int& sl) { t = 0; sl = k; }, 1, stride, a.n_ff, a.h, lane,
                 a.out16 != nullptr);
-    // (a grid of one row chunk has no idle publisher-row workgroup)
-    if (a.sh_gate_w && gridDim.x == 1) shared_gate_tokens(a, tid, kFrontThreads / 32);
     return;
   }
 
@@ -2145,8 +2143,10 @@ __global__ void __launch_bounds__(kBackThreads) layer_back_kernel(LayerArgs args
   back_core<NBF, ROWS, HS, kShapeT != 1>(a, L, dyn, wbuf, row0, nr, res0, hpre, pre);
 }
 
-// The layer's limit on shapes: every token's staged x, the pointer tables and
-// the routing arrays within one workgroup's LDS beside four weight buffers.
+// The shapes that the layer takes: its interface's limit, kept as it was when one
+// workgroup staged every token's x beside the pointer tables, the routing arrays
+// and four weight buffers.  The launches need less (x of several tokens goes
+// through the workspace); what each one needs is checked by itself.
 static bool layer_lds_refused(int T, int nbh, int E, int k) {
   const int teams = T == 1 ? 1 : (T == 2 ? 2 : 4), m = k + 1, e32 = (E + 31) & ~31;
   const int ncp = (4 / teams * m + 3) & ~3, gmax = (T * k < E ? T * k : E) + 1;
@@ -2318,7 +2318,8 @@ static int layer_launch(const sg_block_q4k* const* tab_gate, const sg_block_q4k*
                               : route_lds(n_tokens, n_expert, k).total) * 4;
   const size_t lds_g = static_cast<size_t>((((hidden / kQK) * kXStride + 3) & ~3) + 2 * ws.emax) * 4;
   const int back_bufs = lds_b + kBackWaves * buf_b <= 160 * 1024 ? kBackWaves : 4;
-  if (layer_lds_refused(n_tokens, hidden / kQK, n_expert, k) ||
+  const size_t front_b = lds_f + (one ? 4 * buf_b : 0);  // (one token: beside the static buffers)
+  if (layer_lds_refused(n_tokens, hidden / kQK, n_expert, k) || front_b > 160 * 1024 ||
       lds_b + back_bufs * buf_b > 160 * 1024 || (!one && lds_g + 4 * buf_b > 160 * 1024))
     return set_error(SG_ERR_UNSUPPORTED, "%s: this shape needs more LDS than a workgroup has",
                      nm);

@@ -74,21 +74,33 @@ def test_layer_tokens_one_expert_for_all():
     np.testing.assert_array_equal(out.cpu().numpy().view(np.uint32), ref.view(np.uint32))
 
 
-def test_layer_workspace_of_one_shared_group():
-    """A workspace without room for the split shared expert's extra plan entries
-    (the layout of one group) is enough: the layer takes that layout."""
-    rng = np.random.default_rng(78)
-    H, F, E, k, T = 512, 256, 12, 3, 13
+# (hidden, n_ff, experts, k, tokens, small workspace).  The split shared expert's extra
+# plan entries past a 256-B boundary of the workspace (32 groups against 35: 63744 and
+# 64512 B), or past the back kernel's LDS (163840 B with four row buffers: 163824 B and,
+# exactly, 163840 with one group, 163856 and more with the split)
+ONE_GROUP = [(512, 256, 31, 3, 13, True), (512, 256, 33, 30, 12, False),
+             (1024, 768, 33, 7, 16, False), (512, 512, 12, 11, 16, False)]
+
+
+@pytest.mark.parametrize("H,F,E,k,T,small", ONE_GROUP)
+def test_layer_of_one_shared_group(H, F, E, k, T, small):
+    """Without room for the split shared expert's extra plan entries, in the caller's
+    workspace or in LDS, the layer takes the layout of one shared group."""
+    rng = np.random.default_rng(78 + E)
     mats, sh, layer = _layer(rng, H, F, E, k, T, True)
     x = rng.normal(0, 1, (T, H)).astype(np.float32)
     lg = rng.normal(0, 1, (T, E)).astype(np.float32)
-    al = lambda n: (n + 255) // 256 * 256
-    g, e = min(T * k, E) + 1, T * k + T
-    small = (256 + al(4 * (g + 1)) + 2 * al(4 * e) + 3 * al(8 * g) + al(4 * T)
+    kw = {}
+    if small:
+        al = lambda n: (n + 255) // 256 * 256
+        g, e = min(T * k, E) + 1, T * k + T
+        n = (256 + al(4 * (g + 1)) + 2 * al(4 * e) + 3 * al(8 * g) + al(4 * T)
              + al(4 * T * (k + 1) * F) + al(4 * 80 * T * H // 256))
-    out, idx, w = layer.forward(torch.from_numpy(x).cuda(), torch.from_numpy(lg).cuda(),
-                                workspace=torch.zeros(small, dtype=torch.uint8, device="cuda"))
+        assert n < ops.load().sg_moe_layer_workspace_bytes(T, H, F, E, k)
+        kw["workspace"] = torch.zeros(n, dtype=torch.uint8, device="cuda")
+    out, idx, w = layer.forward(torch.from_numpy(x).cuda(), torch.from_numpy(lg).cuda(), **kw)
     torch.cuda.synchronize()
     ref, ri, _ = orc.moe_layer(mats[0][:E], mats[1][:E], mats[2][:E], sh, x, logits=lg, hidden=H,
                                n_ff=F, k=k)
+    np.testing.assert_array_equal(idx.cpu().numpy()[:, :k], ri[:, :k])
     np.testing.assert_array_equal(out.cpu().numpy().view(np.uint32), ref.view(np.uint32))

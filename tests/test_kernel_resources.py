@@ -7,7 +7,9 @@ decide how they run:
   and a spill in the verify window's gate/up launch made its time erratic
   (35 to 46 us per window between replays);
 - the several-token gate/up launch must fit 128 registers so that four of
-  its workgroups share a CU and its grid runs in one round.
+  its workgroups share a CU and its grid runs in one round; the matrix-core
+  GEMVs (up to sixteen waves) and the prefill's grouped kernels likewise, for
+  four waves per SIMD.
 """
 import concurrent.futures
 import os
@@ -26,10 +28,15 @@ BUDGETS = [
     ("sg_layer.hip", r"layer_front_kernelILi4ELi8ELb0ELi4ELb1E", 0, None),
     ("sg_layer.hip", r"layer_back_kernelILi2ELi8ELi[14]ELb[01]E", 0, None),
     ("sg_layer.hip", r"layer_gateup_kernelILi8ELi4ELb1E", 0, 128),
+    ("sg_layer.hip", r"layer_(front|gateup|back|hq)_kernel", 0, None),
     ("sg_gemv.hip", r"gemv_lat_plain_kernel", 0, None),
+    ("sg_gemv.hip", r"gemv_(mt|mtw)_kernel", 0, 128),
+    ("sg_gemv.hip", r"gemv_batched_kernel", 0, None),
     ("sg_gemv.hip", r"gemv1_kernelINS_9PlainRowsENS_6F32OutELi4E", 0, None),
-    ("sg_prefill.hip", r"grouped_mfma_kernelILb[01]ELb[01]E", 0, None),
+    ("sg_prefill.hip", r"grouped_mfma_kernelILb[01]ELb[01]E", 0, 128),
     ("sg_prefill.hip", r"route_quantize_kernel", 0, None),
+    ("sg_prefill.hip", r"plan_(bits|place)_kernel", 0, None),
+    ("sg_moe.hip", r"gemv_f32_f16x_(tile_)?kernel", 0, None),
     ("sg_q6.hip", r"gemv_q6_kernel", 0, None),
 ]
 

@@ -399,7 +399,8 @@ int sg_moe_dispatch_plan(const int* idx, float* weight, int* gslot, int* grows, 
  * sums are exact int32 (int8 MFMAs); the fp32 epilogue is the
  * integer-first super-block order (t = fma(d, sum sc*ip, -(dmin * sum
  * mn*bsum)), acc = fma(xd, t, acc)).  workspace: at least
- * sg_moe_prefill_workspace_bytes(). */
+ * sg_moe_prefill_workspace_bytes().  The chunk's quantized x, n_tokens *
+ * hidden / 256 * 304 B, is below 2 GiB (else SG_ERR_UNSUPPORTED). */
 size_t sg_moe_prefill_workspace_bytes(int n_tokens, int hidden, int n_ff,
                                       int n_expert, int k);
 int sg_moe_prefill(const sg_block_q4k* const* tab_gate,

@@ -312,6 +312,15 @@ __device__ __forceinline__ bool few_tokens(int nt, int nb) {
   return nt <= kFewTokens && nt * nb <= kFewXRows;
 }
 
+// The Q8P rows that a tile reads by 32-bit offsets (of less than 2 GiB: the range
+// of the descriptor): of any token in the gate/up pass, whose x is within that, of
+// the tile's own consecutive rows from p0 on in the down pass, whose h need not be.
+template <bool kGateUp>
+__device__ __forceinline__ u32x4 x_desc(const GroupedArgs& a, int p0) {
+  return buffer_desc(kGateUp ? a.xq : a.xq + static_cast<long long>(p0) * a.nb * kQ8PBytes,
+                     0x7FFFFFFFu);
+}
+
 // ma: the wave's matrix; slices: column slices from c0 on, in turn
 template <bool kGateUp, bool kF16Out>
 __device__ __forceinline__ void few_tile(const GroupedArgs& a, const sg_block_q4k* mw,
@@ -330,7 +339,7 @@ __device__ __forceinline__ void few_tile(const GroupedArgs& a, const sg_block_q4
   const int pu = __builtin_amdgcn_readfirstlane(p0), nu = __builtin_amdgcn_readfirstlane(nt);
   int rows[kFewTokens];
 #pragma unroll
-  for (int t = 0; t < kFewTokens; ++t) rows[t] = kGateUp ? grows[pu + min(t, nu - 1)] : pu + t;
+  for (int t = 0; t < kFewTokens; ++t) rows[t] = kGateUp ? grows[pu + min(t, nu - 1)] : t;
   const double ev = kGateUp ? kExp2Tab64[lane] : 0.0;
   uint32_t* ring = lds + 4 * wave * kWChunks;
   uint32_t* x = lds + kFewBufs * kWBufWords;
@@ -360,7 +369,7 @@ __device__ __forceinline__ void few_tile(const GroupedArgs& a, const sg_block_q4
   stage(0);
   // the token rows, whole: token t's blocks at x + t nb kXRow
   {
-    const u32x4 rx4 = buffer_desc(a.xq, 0x7FFFFFFFu);
+    const u32x4 rx4 = x_desc<kGateUp>(a, p0);
     const int per = nb * 19, total = nt * per;
 #pragma unroll
     for (int i = 0; i < kFewXInstr; ++i) {
@@ -577,7 +586,7 @@ grouped_mfma_kernel(GroupedArgs a) {
   const int ntb = (nt + 15) >> 4;  // token blocks holding tokens (wave-uniform)
   const int xchunks = ntb * 16 * 19;
   constexpr int kXInstr = (kTokTile * 19 / 64 + 7) / 8;  // per wave: 3
-  const u32x4 rx4 = buffer_desc(a.xq, 0x7FFFFFFFu);
+  const u32x4 rx4 = x_desc<kGateUp>(a, p0);
   uint32_t xofs[kXInstr];
   auto stage_x = [&](int b, int s) {
 #pragma unroll
@@ -591,7 +600,7 @@ grouped_mfma_kernel(GroupedArgs a) {
   if (kGateUp && tid < 64) etab[tid] = kExp2Tab64[tid];  // the SiLU's exp table
   if (tid < kTokTile) {  // block index of each token row (rows past nt repeat the first)
     const int t = tid < nt ? tid : 0;
-    trow[tid] = (kGateUp ? a.grows[t0 + t] : t0 + t) * nb;
+    trow[tid] = (kGateUp ? a.grows[t0 + t] : t) * nb;
   }
   bar();
 #pragma unroll
@@ -1699,6 +1708,10 @@ static int prefill_launch(const sg_block_q4k* const* tab_gate, const sg_block_q4
                      n_tokens, hidden, n_ff);
   if (k <= 0 || k > 32 || n_expert < k || n_expert > 1024)
     return set_error(SG_ERR_GEOMETRY, "%s: k=%d n_expert=%d", nm, k, n_expert);
+  // (x_desc: past this the gate/up pass would read zeros for the last tokens)
+  if (static_cast<long long>(n_tokens) * (hidden / kQK) * kQ8PBytes > 0x7fffffffLL)
+    return set_error(SG_ERR_UNSUPPORTED, "%s: n_tokens=%d x hidden=%d: Q8 of x past 2 GiB", nm,
+                     n_tokens, hidden);
   const PrefillWs ws = prefill_ws(n_tokens, hidden, n_ff, n_expert, k);
   if (workspace_bytes < ws.total)
     return set_error(SG_ERR_INVALID_ARGUMENT, "%s: workspace %zu < %zu bytes", nm,

@@ -55,6 +55,9 @@ def test_validation_without_launch(lib):
     sh = [bad, None, None]
     args2 = [bad] * 3 + sh + [None] + [bad, bad, None, bad, bad, bad, bad]
     assert lib.sg_moe_layer(*args2, ws, 1, 2048, 512, 256, 8, 1.0, None) == 1
+    # a chunk whose Q8 of x (64 blocks of 304 B per token) reaches 2 GiB, and one below
+    assert lib.sg_moe_prefill(*args, 0, 110377, 16384, 512, 8, 2, 1.0, None) == 8
+    assert lib.sg_moe_prefill(*args, 0, 110376, 16384, 512, 8, 2, 1.0, None) == 1  # workspace
     # fp16-buffer launchers and the fp32 x fp16 GEMV reject bad geometry
     assert lib.sg_silu_mul_f16(bad, bad, bad, 0, 512, None) == 4
     assert lib.sg_moe_combine_batched_f16(bad, bad, bad, 8, 2048, 70000, None) == 4

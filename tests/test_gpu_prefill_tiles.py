@@ -100,3 +100,24 @@ def test_few_token_tiles_bit_exact(H, F, T, f16):
         ref = orc.moe_layer(*args, **kw)[0]
     bits = np.uint16 if f16 else np.uint32
     np.testing.assert_array_equal(out.cpu().numpy().view(bits), ref.view(bits))
+
+
+def test_prefill_down_rows_past_2_gib():
+    """A chunk whose Q8 of h passes 2 GiB (110700 positions of 64 super-blocks, 304 B
+    each): its last tokens, and a few at the start, equal a short chunk of the same
+    tokens bit for bit (tokens do not meet)."""
+    rng = np.random.default_rng(3)
+    H, F, T = 256, 16384, 110700
+    mats = [q4k_random_np(rng, F * H // 256) for _ in range(3)]
+    dev = [torch.from_numpy(m).cuda() for m in mats]
+    tabs = [torch.tensor([m.data_ptr()], dtype=torch.int64, device="cuda") for m in dev]
+    x = torch.randn(T, H, device="cuda", generator=torch.Generator("cuda").manual_seed(4))
+    lg = torch.zeros(T, 1, device="cuda")
+
+    def run(xs):
+        pre = ops.MoePrefill(*tabs, None, hidden=H, n_ff=F, n_expert=1, k=1, max_tokens=len(xs))
+        return pre.forward(xs, lg[:len(xs)])[0]
+
+    out = run(x)
+    for part in (slice(0, 200), slice(T - 500, T), slice(T - 5, T)):
+        assert torch.equal(out[part].view(torch.int32), run(x[part].contiguous()).view(torch.int32))

@@ -314,11 +314,12 @@ int sg_moe_layer_f16(const sg_block_q4k* const* tab_gate,
  * harnesses that forbid hipMalloc).  No counterpart in the reference.  The
  * library keeps one 1 MiB scratch array per GPU (a file-scope device array,
  * held until the process ends) and uses it as the workspace; shapes whose
- * sg_moe_layer_workspace_bytes() exceeds 1 MiB are rejected with
- * SG_ERR_UNSUPPORTED (at hidden 2048, n_ff 512, top-8 + shared: up to 16
- * tokens).  Allocates nothing.  Every call on one GPU shares that GPU's
- * array, so calls that overlap on one GPU (two streams, two threads) race:
- * order them on one stream. */
+ * smallest workspace exceeds 1 MiB are rejected with SG_ERR_UNSUPPORTED (at
+ * hidden 2048, n_ff 512, top-8 + shared all of up to 16 tokens fit).  The
+ * smallest one has the shared expert in one group of tokens; it is up to 1 KiB
+ * below sg_moe_layer_workspace_bytes().  Allocates nothing.  Every call on
+ * one GPU shares that GPU's array, so calls that overlap on one GPU (two
+ * streams, two threads) race: order them on one stream. */
 int sg_moe_layer_noalloc(const sg_block_q4k* const* tab_gate,
                          const sg_block_q4k* const* tab_up,
                          const sg_block_q4k* const* tab_down,

@@ -15,7 +15,8 @@
 // Small matrices (up to 262144 super-blocks) take gemv_lat_kernel instead:
 // four lanes per super-block, loads straight into registers, one pass.
 //
-// Several tokens take int8 matrix cores (gemv_mt_kernel, gemv_mtw_kernel).
+// Several tokens take int8 matrix cores (gemv_mt_kernel, gemv_mtw_kernel), two to
+// four of them in some large matrices the sdot4 kernel (use_batched_sdot).
 //
 // Reference kernels replaced: gemv_q4_k_q8 / gemv_mtok_ro_f32_kernel
 // (q4_k.cu:57-91, 1360-1422, 1534-1562), gemv_q4_k_q8_batched and the mtok
@@ -554,7 +555,7 @@ __global__ void __launch_bounds__(64 * kMtWaves) gemv_mt_kernel(
 // in rows 8j..8j+7 of its A operand, zero elsewhere, and the two groups' MFMAs
 // accumulate into one result whose row half j is group j's.
 //
-// Bound by the weight stream: 248320 x 2048 x 4 tokens 77.6 -> 54.8 us (5.3
+// Bound by the weight stream: 248320 x 2048 x 4 tokens 77.6 -> 54.8 us (5.2
 // TB/s).  With 64-row sets loaded straight to registers it took 70 us: 16-B
 // pieces of a 128-B line asked for by several instructions, against whole
 // lines here.

@@ -1580,7 +1580,9 @@ layer_gateup_kernel(LayerArgs args) {
 // blocks whole before it writes, and block e's Q8_K (kXStride words, the LDS
 // layout) takes the head of its 1024 B.  The line, per layer, in the back
 // kernel / by the launch: hidden 2048, 36 blocks 26.2 / 26.7 us, 54 29.7 / 29.9,
-// 90 39.1 / 37.2, 288 79.6 / 65.6; hidden 1280, 48 blocks 37.9 / 35.3.
+// 90 39.1 / 37.2, 288 79.6 / 65.6; hidden 1280, 48 blocks 37.9 / 35.3.  It depends
+// on hidden, so one line is a compromise: at hidden 2048 the two are equal at 54,
+// at 1280 the launch is ahead at 48 already.
 constexpr int kHqBlocks = 48;
 static_assert(kShapeWindow * (kShapeK + 1) * (kShapeFf / kQK) >= kHqBlocks,
               "the window's instances take h quantized");

@@ -7,20 +7,20 @@
 //   plan (moe.cu:366-444) -> grouped gate/up + SiLU -> Q8_K(h) -> grouped
 //   down -> combine in slot order (moe.cu:265-280).
 //
-// The grouped contractions run on v_mfma_i32_16x16x32_i8: one MFMA is one
-// Q4_K sub-block (32 weights) for 16 tokens x 16 weight rows, so every
-// int32 sub-block dot is exact.  Per super-block each output keeps
-// I = sum_s sc_s * ip_s and M = sum_s mn_s * bsum_s as exact integers; the
-// fp32 epilogue is t = fma(d, I, -(dmin * M)), acc = fma(xd, t, acc) over
-// the super-blocks in order (the integer-first order; the CPU oracle's
-// orc_gemv_q4k_q8_int is the same arithmetic).
+// The grouped contractions run on v_mfma_i32_16x16x64_i8, exactly: per
+// super-block each output keeps I = sum_s sc_s * ip_s and M = sum_s mn_s *
+// bsum_s as integers (the scales folded into the weight operand, or in tiles
+// of a few tokens applied to each sub-block's dot); the fp32 epilogue is t =
+// fma(d, I, -(dmin * M)), acc = fma(xd, t, acc) over the super-blocks in order
+// (the integer-first order; the CPU oracle's orc_gemv_q4k_q8_int is the same
+// arithmetic).
 //
 // Workgroup tile: up to 96 tokens x 128 weight rows (gate/up: 64 h rows of gate
-// and the same 64 of up; down: 128 output rows), eight waves of 16 tokens x
-// 64 rows each (gate/up: 32 h rows of gate and their up rows, so SiLU pairs
-// meet in one lane), K streamed one super-block at a time through two LDS
-// buffers (weights by global_load_lds, token rows gathered through
-// registers).
+// and the same 64 of up; down: 128 output rows), eight waves of 16 weight rows
+// each, which take the tile's 16-token blocks in turn (gate/up: waves 0-3 gate,
+// 4-7 up, halves of the tokens exchanged for the SiLU).  K is streamed one
+// super-block at a time with buffer_load ... lds: the token rows through two
+// LDS buffers, the weights through one, whose 16 rows each wave refills itself.
 #include <cmath>
 
 #include "sg_common.hpp"

@@ -369,8 +369,8 @@ int sg_moe_dispatch_scan(const int* idx, float* weight, int* gslot, int* grows,
                          int n_expert, int tok_per, void* stream);
 
 /* The same plan built over many workgroups (32 tokens each: bitmaps, then
- * offsets and placement; one launch up to 512 rows, else two), with no
- * limit on n_rows beyond int indexing; the order inside an expert is the
+ * offsets and placement; one launch for up to 512 rows of few routes, else
+ * two), with no limit on n_rows beyond int indexing; the order inside an expert is the
  * same (token, then slot), so every array equals sg_moe_dispatch_scan's.
  * It is the plan sg_moe_prefill builds.  Extra outputs:
  *   shared_tail: the shared expert's rows (0 = none, else n_rows) appended

@@ -814,9 +814,9 @@ grouped_mfma_kernel(GroupedArgs a) {
 //    and the tile records.  A row with a duplicated id (caller routing only)
 //    is placed serially in (token, slot) order by workgroup 0 alone, as
 //    dispatch_scan_kernel does.
-// Up to kPlanFusedRows tokens the first launch is left out: every workgroup of
-// the second builds all the bitmaps itself, in LDS, from the ids (a chunk of 57
-// tokens 134.7 -> 130.7 us, of 512 174.5 -> 173.0).
+// For few tokens and routes (plan_fused) the first launch is left out: every
+// workgroup of the second builds all the bitmaps itself, in LDS, from the ids (a
+// chunk of 57 tokens 134.7 -> 130.7 us, of 512 174.5 -> 173.0).
 constexpr int kPlanThreads = 512;
 constexpr int kPlanMaxWg = 256;   // bitmap workgroups; m grows with T beyond 256 * 32 tokens
 
@@ -878,6 +878,20 @@ __global__ void __launch_bounds__(kPlanThreads) plan_bits_kernel(
 // in workgroup 0, the experts' matrix pointers.
 constexpr int kColWords = 32;  // bitmap words of one expert's column per thread
 constexpr int kPlanFusedRows = 512;
+// Each of its workgroups sets a bit per route and clears, then counts, a word per
+// expert and 32 tokens, about 64 (expert, token) pairs to a route's time; the two
+// launches take 11.5 to 13 us whatever the routes, from 513 experts on (two passes)
+// 14 to 15.  Both plans (us, two launches / one), by routes + pairs / 64: 256
+// experts, 512 tokens, top 8 (6144) 11.9 / 9.3, top 16 (10240) 12.1 / 11.8, top 24
+// (14336) 12.2 / 14.6; 512, 512, top 12 (10240) 12.1 / 12.0, top 16 12.0 / 13.2;
+// 1024, 384, top 24 (15360) 15.4 / 14.1, 512, top 16 (16384) 15.4 / 15.9, top 32
+// 15.9 / 21.1; 700, 512, top 12 (11744) 14.0 / 13.5, top 16 (13792) 14.1 / 14.8.  Up to 32
+// experts the two launches are slower (many routes to a word: 24 experts, 512
+// tokens, top 24 15.3 / 14.8).
+static bool plan_fused(int n_rows, int k, int E) {
+  if (n_rows > kPlanFusedRows) return false;
+  return E <= 32 || n_rows * k + E * n_rows / 64 <= 10240 + (E > 512 ? 5 * E : 0);
+}
 
 // kFused: no plan_bits_kernel before it (m = 1; wbits and wflags unused)
 template <bool kFused>
@@ -1581,7 +1595,7 @@ static int plan_launch(const int* idx, float* weight, int* gslot, int* grows, in
                        gslot, grows, off, toff, meta, tiles, trec, n_rec, pt.g, pt.u, pt.d, pt.sg,
                        pt.su, pt.sd, n_rows, k, E, p.m, p.n_w, tok_per, shared_tail);
   };
-  if (n_rows <= kPlanFusedRows) {
+  if (plan_fused(n_rows, k, E)) {
     place(plan_place_kernel<true>, static_cast<size_t>(E) * p.n_w * 4);
     return check_launch(nm);
   }

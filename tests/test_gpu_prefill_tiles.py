@@ -41,11 +41,15 @@ def test_prefill_tiles_bit_exact(H, F, E, k, T, shared):
 
 @pytest.mark.parametrize("n_rows,E,k,dup", [(1, 8, 2, False), (31, 700, 32, False),
                                             (512, 1024, 32, False), (512, 61, 5, True),
-                                            (513, 61, 5, False), (32, 5, 5, False)])
+                                            (513, 61, 5, False), (32, 5, 5, False),
+                                            (512, 1024, 14, False), (512, 1024, 15, True),
+                                            (512, 256, 16, True), (512, 256, 17, True),
+                                            (512, 32, 32, False), (512, 33, 20, False)])
 def test_plan_of_one_launch(n_rows, E, k, dup):
-    """Up to 512 rows the plan is one launch: every array against the oracle's scan,
-    with invalid ids and (dup) a row that names an expert twice, at its last row
-    count and the two-launch form's first, more and fewer experts than threads,
+    """For up to 512 rows of few routes the plan is one launch: every array against
+    the oracle's scan, with invalid ids and (dup) a row that names an expert twice, at
+    its last row count and the two-launch form's first, at its last route counts
+    and one past them (up to 32 experts all), more and fewer experts than threads,
     and a full and a partial last group of 32 rows."""
     rng = np.random.default_rng(n_rows + E)
     idx = np.stack([rng.choice(E, k, replace=False) for _ in range(n_rows)]).astype(np.int32)

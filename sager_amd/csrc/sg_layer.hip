@@ -1503,7 +1503,10 @@ layer_front_kernel(LayerArgs args) {
 // left in the workspace: several tokens (a verify window), where routing in
 // every compute workgroup would cost more than a launch.  Grid (row chunks
 // of 16, gmax); groups beyond the plan's count exit.
-template <int NBH, int kShapeT = 0, bool kSh = false, int kIo = 0>
+// kWide: hidden past 7168, where x is more than the 576 16-B chunks of nine copy
+// instructions (hidden 8192: 640).  An instance of its own: with the tenth in
+// every one the batch of 11 tokens at hidden 7168 took 2 % longer.
+template <int NBH, int kShapeT = 0, bool kSh = false, int kIo = 0, bool kWide = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
 layer_gateup_kernel(LayerArgs args) {
   LayerArgs a = args;
@@ -1545,11 +1548,8 @@ layer_gateup_kernel(LayerArgs args) {
     const int t0 = ent1 ? __shfl(v_tok, j0, 64) : a.plan.tok[j0];
     const uint32_t* src = a.xq + static_cast<long long>(t0) * xw;
     dma_chunks([&](int c) { return reinterpret_cast<const char*>(src) + 16 * c; },
-               min(xw / 4, 576), x0, lane, wave, 4);
-    // past hidden 7168 x is more than the 576 chunks of nine instructions: a
-    // tenth, wave 1's turn (hidden <= 8192: 640 chunks).  One loop over all
-    // chunks instead made the batch of 13 tokens 3 % slower.
-    if (NBH == 0 && wave == 1 && 576 + lane < xw / 4)
+               kWide ? 576 : xw / 4, x0, lane, wave, 4);
+    if (kWide && wave == 1 && 576 + lane < xw / 4)
       __builtin_amdgcn_global_load_lds((glb_void_p)(src + 4 * (576 + lane)),
                                        (lds_void_p)(x0 + 4 * 576), 16, 0, 0);
   }
@@ -2416,6 +2416,8 @@ static int layer_launch(const sg_block_q4k* const* tab_gate, const sg_block_q4k*
                            a);
       else if (hidden / kQK == 8)
         hipLaunchKernelGGL((layer_gateup_kernel<8>), gg, dim3(256), lds_g, s, a);
+      else if (hidden > 28 * kQK)
+        hipLaunchKernelGGL((layer_gateup_kernel<0, 0, false, 0, true>), gg, dim3(256), lds_g, s, a);
       else
         hipLaunchKernelGGL((layer_gateup_kernel<0>), gg, dim3(256), lds_g, s, a);
       if (int st = check_launch("sg_moe_layer/gateup")) return st;
